@@ -373,7 +373,7 @@ int sgpu_gpt2_forward_stages(sgpu_gpt2 *e, int token, int pos, float *logits_hos
  * filled, the final rows left in xT.  Attention: the reference's per-row launches (k/v copies,
  * scores, softmax, mix for each row), or -- with the cache within 8192 positions -- two
  * strided copies of every row's k and v into the caches and one launch of the batched causal
- * attention (one block per head and row, same arithmetic as the fused decode attention). */
+ * attention. */
 static int prefill_layers(sgpu_gpt2 *e, const int *ids, int T) {
     const sgpu_gpt2_cfg *c = &e->cfg;
     const int C = c->C, FC = c->FC;

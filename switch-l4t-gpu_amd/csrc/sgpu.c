@@ -1626,8 +1626,8 @@ int sgpu_internal_pf_attn(const float *qkv, const float *kc, const float *vc, fl
     devstate *d = cur(&rc);
     if (!d) return rc;
     int QKVD = (NH + 2 * NKV) * HD;
-    unsigned g[3] = {(unsigned)NH, (unsigned)T, 1}, b[3] = {256, 1, 1};
-    void *args[] = {(void *)&qkv, (void *)&kc, (void *)&vc, (void *)&out, &pos0, &NH, &NKV, &scale, &QKVD};
+    unsigned g[3] = {(unsigned)NH * cdiv(T, 32), 1, 1}, b[3] = {256, 1, 1};   /* a block per head and 32 rows */
+    void *args[] = {(void *)&qkv, (void *)&kc, (void *)&vc, (void *)&out, &pos0, &T, &NH, &NKV, &scale, &QKVD};
     return launch(d->pf_attn[j], g, b, stream, args);
 }
 

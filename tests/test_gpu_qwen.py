@@ -246,6 +246,23 @@ def test_engine_prefill_matches_golden(gpu, og, case):
     eng.close()
 
 
+# The causal attention's tiles: 32 query rows a block, 32 keys a tile, tiles dealt to four waves.
+@pytest.mark.parametrize("T", [31, 32, 33, 127, 161])
+@pytest.mark.parametrize("heads", [(4, 2, 32), (6, 1, 64), (2, 2, 128)], ids=["hd32", "hd64", "hd128"])
+def test_engine_prefill_attention_tiles(gpu, og, heads, T):
+    NH, NKV, HD = heads
+    cfg = dict(V=300, C=NH * HD, NL=2, NH=NH, NKV=NKV, HD=HD, FC=256, CTX=200)
+    test_engine_prefill_matches_golden(gpu, og, dict(cfg=cfg, T=T))
+    # rows that a longer prompt left in the cache are not read
+    blob = gpu.qwen_random_blob(gpu.qwen_cfg(**cfg), seed=52, std=0.15)
+    used, fresh = (gpu.QwenEngine(gpu.qwen_cfg(**cfg), blob, PATHS["fused"]) for _ in range(2))
+    ids = [int(v) for v in np.random.default_rng(T).integers(0, cfg["V"], 200)]
+    used.prefill(ids)
+    assert np.array_equal(used.prefill(ids[:T]), fresh.prefill(ids[:T]))
+    used.close()
+    fresh.close()
+
+
 def test_engine_prefill_rejects_bad_ids(gpu):
     cfg = SMALL
     eng = gpu.QwenEngine(gpu.qwen_cfg(**cfg), gpu.qwen_random_blob(gpu.qwen_cfg(**cfg), seed=3), PATHS["fused"])
