@@ -397,7 +397,7 @@ static int prefill_layers(sgpu_gpt2 *e, const int *ids, int T) {
                 he = hipMemcpy2DAsync(e->vc[l], row, e->qkvT + 2 * C, qrow, row, (size_t)T, hipMemcpyDeviceToDevice,
                                       e->stream);
             if (he != hipSuccess) return (int)he;
-            TRY(sgpu_internal_pf_attn(e->qkvT, e->kc[l], e->vc[l], e->attT, T, 0, c->NH, c->NH, c->HD, scale, s));
+            TRY(sgpu_internal_pf_attn(e->qkvT, e->kc[l], e->vc[l], e->attT, NULL, NULL, T, 0, c->NH, c->NH, c->HD, scale, s));
         } else {
             for (int t = 0; t < T; t++) {     /* causal attention, one query row at a time */
                 const float *qrow = e->qkvT + (size_t)t * 3 * C;

@@ -49,6 +49,11 @@ static int cfg_ok(const sgpu_qwen_cfg *c) {
            (long long)c->CTX * c->NH < 0x7fffffffLL;
 }
 
+/* sizes the fused decode and prefill kernels take */
+static int fused_ok(const sgpu_qwen_cfg *c) {
+    return c->CTX <= 8192 && (c->HD == 32 || c->HD == 64 || c->HD == 128) && c->C % 8 == 0 && c->FC % 8 == 0;
+}
+
 void sgpu_qwen_default_cfg(sgpu_qwen_cfg *c) {
     /* qwen_engine.c:43-55, conv_qwen.py:23-27 */
     c->V = 151936; c->C = 896; c->NL = 24; c->NH = 14; c->NKV = 2; c->HD = 64; c->FC = 4864;
@@ -115,6 +120,9 @@ struct sgpu_qwen {
     unsigned *d_split_cnt;                     /* ... and per-tile counters (kept at zero) */
     int *d_pf_ids;                             /* batched prefill: prompt ids and row buffers */
     float *d_pf_x, *d_pf_xn, *d_pf_qkv, *d_pf_att, *d_pf_y, *d_pf_g;
+    int mm_rows;                               /* rows the piece buffers below hold */
+    float *d_mm_x, *d_mm_qkv, *d_mm_ws;        /* ... and the split-K partials */
+    uint16_t *d_mm_xn, *d_mm_att, *d_mm_g;     /* fp16 pieces and, after them, their scales */
     hipGraph_t g_layers, g_step;
     hipGraphExec_t ge_layers, ge_step;
     uint16_t *d_emb, *d_lnfw;
@@ -130,6 +138,8 @@ static int dalloc(void **p, size_t bytes, const void *src) {
     if (src) return sgpu_memcpy_htod(*p, src, bytes);
     return sgpu_memset_d8(*p, 0, bytes);
 }
+
+static void mm_free(sgpu_qwen *e);
 
 void sgpu_qwen_destroy(sgpu_qwen *e) {
     if (!e) return;
@@ -167,6 +177,7 @@ void sgpu_qwen_destroy(sgpu_qwen *e) {
     sgpu_free(e->d_pf_ids);
     float *pf[] = {e->d_pf_x, e->d_pf_xn, e->d_pf_qkv, e->d_pf_att, e->d_pf_y, e->d_pf_g};
     for (size_t i = 0; i < sizeof pf / sizeof pf[0]; i++) sgpu_free(pf[i]);
+    mm_free(e);
     if (e->stream) hipStreamDestroy(e->stream);
     free(e);
 }
@@ -217,6 +228,14 @@ int sgpu_qwen_create(sgpu_qwen **out, const sgpu_qwen_cfg *c, const void *blob) 
         }
         free(tmp);
         if (rc) goto fail;
+        /* the layers' subnormal weight codes become the zeros they are read as, which the fp16
+         * matrix cores (prefill) would not do themselves */
+        for (int l = 0; l < NL && fused_ok(c); l++) {
+            TRY(sgpu_internal_h16_flush(e->d_qkvw[l], (size_t)QKVD * C, (void *)e->stream));
+            TRY(sgpu_internal_h16_flush(e->d_ow[l], (size_t)C * C, (void *)e->stream));
+            TRY(sgpu_internal_h16_flush(e->d_gateupw[l], (size_t)2 * FC * C, (void *)e->stream));
+            TRY(sgpu_internal_h16_flush(e->d_downw[l], (size_t)C * FC, (void *)e->stream));
+        }
     }
     TRY(dalloc((void **)&e->d_x, (size_t)C * 4, NULL));
     TRY(dalloc((void **)&e->d_ln1, (size_t)C * 4, NULL));
@@ -311,10 +330,6 @@ static int forward_reference(sgpu_qwen *e, int token, int pos, int want_logits, 
 }
 
 /* ---- fused path: five kernels per layer (sgpu_decode.hip) ---- */
-static int fused_ok(const sgpu_qwen_cfg *c) {
-    return c->CTX <= 8192 && (c->HD == 32 || c->HD == 64 || c->HD == 128) && c->C % 8 == 0 && c->FC % 8 == 0;
-}
-
 static int fused_layers(sgpu_qwen *e) {
     const sgpu_qwen_cfg *c = &e->cfg;
     const int C = c->C, NH = c->NH, NKV = c->NKV, HD = c->HD, FC = c->FC, QKVD = e->L.qkvd;
@@ -497,8 +512,20 @@ int sgpu_qwen_phase_times(sgpu_qwen *e, int pos, int reps, float *us) {
 }
 
 /* ---- batched prompt prefill: the prompt's rows go through each layer together, so each
- * layer's weights stream once per chunk of up to PF_ROWS rows instead of once per position ---- */
+ * layer's weights stream once per chunk of rows instead of once per position.  Two forms:
+ *  * products in fp16 pieces (sgpu_prefill.hip), chunks of up to MM_ROWS rows;
+ *  * fp32 MFMA tiles of 32 rows (sgpu_pf_gemm), chunks of up to PF_ROWS rows: for prompts of up
+ *    to MM_MIN_ROWS rows and for head or layer sizes that are no whole 64-blocks. ---- */
 #define PF_ROWS 512
+#define MM_ROWS 4096
+#define MM_MIN_ROWS 64
+
+static int mm_ok(const sgpu_qwen_cfg *c) {
+    const long long wide = c->FC > c->C ? c->FC : c->C;
+    return (c->HD == 64 || c->HD == 128) && c->NH * c->HD == c->C && c->C % 64 == 0 && c->FC % 64 == 0 &&
+           3LL * MM_ROWS * wide < 1LL << 30 && 2 * wide * c->C < 1LL << 30 &&
+           (long long)(c->C + 2 * c->NKV * c->HD) * c->C < 1LL << 30;
+}
 
 /* Allocated on the first prefill and kept; a failed call leaves the buffers it did get in
  * place (freed with the engine) and the next call allocates only the missing ones. */
@@ -507,7 +534,7 @@ static int pf_alloc(sgpu_qwen *e) {
     const size_t R = PF_ROWS, C = (size_t)c->C, FC = (size_t)c->FC, Q = (size_t)e->L.qkvd;
     const size_t ybig = 2 * FC > C ? 2 * FC : C;
     struct { void **p; size_t bytes; } need[] = {
-        {(void **)&e->d_pf_ids, (size_t)c->CTX * sizeof(int)}, {(void **)&e->d_pf_x, R * C * 4},
+        {(void **)&e->d_pf_x, R * C * 4},
         {(void **)&e->d_pf_xn, R * C * 4}, {(void **)&e->d_pf_qkv, R * Q * 4}, {(void **)&e->d_pf_att, R * C * 4},
         {(void **)&e->d_pf_y, R * ybig * 4}, {(void **)&e->d_pf_g, R * FC * 4}};
     for (size_t i = 0; i < sizeof need / sizeof need[0]; i++) {
@@ -522,47 +549,119 @@ static int pf_alloc(sgpu_qwen *e) {
     return SGPU_OK;
 }
 
-/* Positions 0..T-1 of the prompt into the KV caches, the last row's logits into d_logits and
- * the step record {ids[T-1], T-1} (so the on-device greedy loop continues from position T). */
-static int prefill_rows(sgpu_qwen *e, const int *ids, int T) {
+/* The piece form's buffers for `rows` rows, kept for later prompts of up to as many.  Every
+ * value a kernel reads there was written by the same prefill, so they are not cleared. */
+static void mm_free(sgpu_qwen *e) {
+    void **p[] = {(void **)&e->d_mm_x, (void **)&e->d_mm_qkv, (void **)&e->d_mm_ws,
+                  (void **)&e->d_mm_xn, (void **)&e->d_mm_att, (void **)&e->d_mm_g};
+    for (size_t i = 0; i < sizeof p / sizeof p[0]; i++) {
+        sgpu_free(*p[i]);
+        *p[i] = NULL;
+    }
+    e->mm_rows = 0;
+}
+static size_t mm_codes(size_t rows, size_t K) { return 3 * rows * K; }
+static float *mm_scales(const sgpu_qwen *e, uint16_t *P, size_t K) { return (float *)(P + mm_codes((size_t)e->mm_rows, K)); }
+static int mm_alloc(sgpu_qwen *e, int rows) {
+    if (rows <= e->mm_rows) return SGPU_OK;
+    const size_t R = (size_t)rows, C = (size_t)e->cfg.C, FC = (size_t)e->cfg.FC, Q = (size_t)e->L.qkvd;
+    int rc = sgpu_stream_synchronize((void *)e->stream);
+    if (rc) return rc;
+    mm_free(e);
+    const size_t xb = mm_codes(R, C) * 2 + R * (C / 64) * 4, gb = mm_codes(R, FC) * 2 + R * (FC / 64) * 4;
+    if ((rc = sgpu_malloc((void **)&e->d_mm_x, R * C * 4)) || (rc = sgpu_malloc((void **)&e->d_mm_qkv, R * Q * 4)) ||
+        (rc = sgpu_malloc((void **)&e->d_mm_ws, (size_t)SGPU_PF_WS_FLOATS * 4)) ||
+        (rc = sgpu_malloc((void **)&e->d_mm_xn, xb)) || (rc = sgpu_malloc((void **)&e->d_mm_att, xb)) ||
+        (rc = sgpu_malloc((void **)&e->d_mm_g, gb))) {
+        mm_free(e);
+        return rc;
+    }
+    e->mm_rows = rows;
+    return SGPU_OK;
+}
+
+#define TRY(x) do { if ((rc = (x))) return rc; } while (0)
+/* The layers over prompt rows c0..c0+Tc-1 in fp16 pieces; the rows' last residual is left in d_mm_x. */
+static int mm_chunk(sgpu_qwen *e, int c0, int Tc) {
+    const sgpu_qwen_cfg *c = &e->cfg;
+    const int C = c->C, NH = c->NH, NKV = c->NKV, HD = c->HD, FC = c->FC, QKVD = e->L.qkvd;
+    const float eps = c->eps, scale = (float)(1.0 / sqrt((double)HD));
+    float *xd = mm_scales(e, e->d_mm_xn, (size_t)C), *ad = mm_scales(e, e->d_mm_att, (size_t)C);
+    float *gd = mm_scales(e, e->d_mm_g, (size_t)FC);
+    void *s = (void *)e->stream;
+    int rc;
+    TRY(sgpu_internal_pf_embed(e->d_emb, e->d_pf_ids + c0, Tc, e->d_mm_x, C, s));
+    for (int l = 0; l < c->NL; l++) {
+        TRY(sgpu_internal_pf_rms(e->d_mm_x, e->d_ln1w[l], e->d_mm_xn, xd, C, eps, Tc, s));
+        TRY(sgpu_internal_pf_mm(e->d_qkvw[l], e->d_mm_xn, xd, e->d_qkvb[l], e->d_mm_qkv, C, QKVD, Tc, e->d_mm_ws,
+                                e->d_split_cnt, 0, s));
+        TRY(sgpu_internal_pf_qkv_post(e->d_mm_qkv, Tc, c0, e->d_cos, e->d_sin, e->d_kc[l], e->d_vc[l], NH, NKV, HD, s));
+        TRY(sgpu_internal_pf_attn(e->d_mm_qkv, e->d_kc[l], e->d_vc[l], NULL, e->d_mm_att, ad, Tc, c0, NH, NKV, HD, scale,
+                                  s));
+        TRY(sgpu_internal_pf_mm(e->d_ow[l], e->d_mm_att, ad, NULL, e->d_mm_x, C, C, Tc, e->d_mm_ws, e->d_split_cnt, 1, s));
+        TRY(sgpu_internal_pf_rms(e->d_mm_x, e->d_ln2w[l], e->d_mm_xn, xd, C, eps, Tc, s));
+        TRY(sgpu_internal_pf_gateup(e->d_gateupw[l], e->d_mm_xn, xd, e->d_mm_g, gd, C, FC, Tc, s));
+        TRY(sgpu_internal_pf_mm(e->d_downw[l], e->d_mm_g, gd, NULL, e->d_mm_x, FC, C, Tc, e->d_mm_ws, e->d_split_cnt, 1, s));
+    }
+    return SGPU_OK;
+}
+
+/* ... and on fp32 MFMA tiles, the last residual in d_pf_x. */
+static int pf_chunk(sgpu_qwen *e, int c0, int Tc) {
     const sgpu_qwen_cfg *c = &e->cfg;
     const int C = c->C, NH = c->NH, NKV = c->NKV, HD = c->HD, FC = c->FC, QKVD = e->L.qkvd;
     const float eps = c->eps, scale = (float)(1.0 / sqrt((double)HD));
     void *s = (void *)e->stream;
     int rc;
-    if ((rc = pf_alloc(e))) return rc;
+    TRY(sgpu_internal_pf_embed(e->d_emb, e->d_pf_ids + c0, Tc, e->d_pf_x, C, s));
+    for (int l = 0; l < c->NL; l++) {
+        TRY(sgpu_rmsnorm(e->d_pf_x, e->d_ln1w[l], e->d_pf_xn, C, eps, Tc, s));
+        TRY(sgpu_internal_pf_gemm(e->d_qkvw[l], e->d_pf_xn, e->d_qkvb[l], e->d_pf_qkv, C, QKVD, Tc,
+            e->d_split_ws, e->d_split_cnt, 0, s));
+        TRY(sgpu_internal_pf_qkv_post(e->d_pf_qkv, Tc, c0, e->d_cos, e->d_sin, e->d_kc[l], e->d_vc[l], NH, NKV,
+                                      HD, s));
+        TRY(sgpu_internal_pf_attn(e->d_pf_qkv, e->d_kc[l], e->d_vc[l], e->d_pf_att, NULL, NULL, Tc, c0, NH, NKV, HD,
+                                  scale, s));
+        /* x += o(att): the residual add in the GEMM's store (x + y, as add2 computes it) */
+        TRY(sgpu_internal_pf_gemm(e->d_ow[l], e->d_pf_att, NULL, e->d_pf_x, C, C, Tc,
+            e->d_split_ws, e->d_split_cnt, 1, s));
+        TRY(sgpu_rmsnorm(e->d_pf_x, e->d_ln2w[l], e->d_pf_xn, C, eps, Tc, s));
+        TRY(sgpu_internal_pf_gemm(e->d_gateupw[l], e->d_pf_xn, NULL, e->d_pf_y, C, 2 * FC, Tc,
+            e->d_split_ws, e->d_split_cnt, 0, s));
+        TRY(sgpu_internal_pf_swiglu(e->d_pf_y, e->d_pf_g, FC, Tc, s));
+        TRY(sgpu_internal_pf_gemm(e->d_downw[l], e->d_pf_g, NULL, e->d_pf_x, FC, C, Tc,
+            e->d_split_ws, e->d_split_cnt, 1, s));
+    }
+    return SGPU_OK;
+}
+
+/* Positions 0..T-1 of the prompt into the KV caches, the last row's logits into d_logits and
+ * the step record {ids[T-1], T-1} (so the on-device greedy loop continues from position T). */
+static int prefill_rows(sgpu_qwen *e, const int *ids, int T) {
+    const sgpu_qwen_cfg *c = &e->cfg;
+    const int C = c->C, mm = T > MM_MIN_ROWS && mm_ok(c);
+    /* equal chunks (of whole 128-row tiles in the piece form) */
+    const int nchunk = mm ? (T + MM_ROWS - 1) / MM_ROWS : 1;
+    const int R = mm ? ((T + nchunk - 1) / nchunk + 127) / 128 * 128 : PF_ROWS;
+    void *s = (void *)e->stream;
+    int rc;
+    if (!e->d_pf_ids) TRY(sgpu_malloc((void **)&e->d_pf_ids, (size_t)c->CTX * sizeof(int)));
+    TRY(mm ? mm_alloc(e, (R + 511) / 512 * 512) : pf_alloc(e));
     hipError_t he = hipMemcpyAsync(e->d_pf_ids, ids, (size_t)T * sizeof(int), hipMemcpyHostToDevice, e->stream);
     if (he != hipSuccess) return (int)he;
-#define TRY(x) do { if ((rc = (x))) return rc; } while (0)
     int Tc = 0;
-    for (int c0 = 0; c0 < T; c0 += PF_ROWS) {
-        Tc = T - c0 < PF_ROWS ? T - c0 : PF_ROWS;
-        TRY(sgpu_internal_pf_embed(e->d_emb, e->d_pf_ids + c0, Tc, e->d_pf_x, C, s));
-        for (int l = 0; l < c->NL; l++) {
-            TRY(sgpu_rmsnorm(e->d_pf_x, e->d_ln1w[l], e->d_pf_xn, C, eps, Tc, s));
-            TRY(sgpu_internal_pf_gemm(e->d_qkvw[l], e->d_pf_xn, e->d_qkvb[l], e->d_pf_qkv, C, QKVD, Tc,
-                e->d_split_ws, e->d_split_cnt, 0, s));
-            TRY(sgpu_internal_pf_qkv_post(e->d_pf_qkv, Tc, c0, e->d_cos, e->d_sin, e->d_kc[l], e->d_vc[l], NH, NKV,
-                                          HD, s));
-            TRY(sgpu_internal_pf_attn(e->d_pf_qkv, e->d_kc[l], e->d_vc[l], e->d_pf_att, Tc, c0, NH, NKV, HD, scale, s));
-            /* x += o(att): the residual add in the GEMM's store (x + y, as add2 computes it) */
-            TRY(sgpu_internal_pf_gemm(e->d_ow[l], e->d_pf_att, NULL, e->d_pf_x, C, C, Tc,
-                e->d_split_ws, e->d_split_cnt, 1, s));
-            TRY(sgpu_rmsnorm(e->d_pf_x, e->d_ln2w[l], e->d_pf_xn, C, eps, Tc, s));
-            TRY(sgpu_internal_pf_gemm(e->d_gateupw[l], e->d_pf_xn, NULL, e->d_pf_y, C, 2 * FC, Tc,
-                e->d_split_ws, e->d_split_cnt, 0, s));
-            TRY(sgpu_internal_pf_swiglu(e->d_pf_y, e->d_pf_g, FC, Tc, s));
-            TRY(sgpu_internal_pf_gemm(e->d_downw[l], e->d_pf_g, NULL, e->d_pf_x, FC, C, Tc,
-                e->d_split_ws, e->d_split_cnt, 1, s));
-        }
+    for (int c0 = 0; c0 < T; c0 += R) {
+        Tc = T - c0 < R ? T - c0 : R;
+        TRY(mm ? mm_chunk(e, c0, Tc) : pf_chunk(e, c0, Tc));
     }
-    TRY(sgpu_internal_dec_lmhead(e->d_emb, C, c->V, e->d_pf_x + (size_t)(Tc - 1) * C, e->d_lnfw, eps, e->d_logits, s));
-#undef TRY
+    TRY(sgpu_internal_dec_lmhead(e->d_emb, C, c->V, (mm ? e->d_mm_x : e->d_pf_x) + (size_t)(Tc - 1) * C, e->d_lnfw,
+                                 c->eps, e->d_logits, s));
     const int st[2] = {ids[T - 1], T - 1};
     he = hipMemcpyAsync(e->d_step, st, sizeof st, hipMemcpyHostToDevice, e->stream);
     if (he != hipSuccess) return (int)he;
     return sgpu_stream_synchronize(s);
 }
+#undef TRY
 
 int sgpu_qwen_prefill(sgpu_qwen *e, const int *ids, int T, float *logits_host) {
     if (!e || !ids || T <= 0 || T > e->cfg.CTX || !fused_ok(&e->cfg)) return SGPU_ERR_INVALID_ARG;

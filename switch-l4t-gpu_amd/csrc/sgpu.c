@@ -28,9 +28,10 @@ extern const unsigned char sgpu_co_gpt2_kernels[], sgpu_co_gpt2_kernels_end[];
 extern const unsigned char sgpu_co_qwen_kernels[], sgpu_co_qwen_kernels_end[];
 extern const unsigned char sgpu_co_sgpu_tuned[], sgpu_co_sgpu_tuned_end[];
 extern const unsigned char sgpu_co_sgpu_decode[], sgpu_co_sgpu_decode_end[];
+extern const unsigned char sgpu_co_sgpu_prefill[], sgpu_co_sgpu_prefill_end[];
 extern const unsigned char sgpu_co_sgpu_probe[], sgpu_co_sgpu_probe_end[];
 
-enum { MOD_SWITCH, MOD_GEMV, MOD_GPT2, MOD_QWEN, MOD_TUNED, MOD_DECODE, MOD_PROBE, NMOD };
+enum { MOD_SWITCH, MOD_GEMV, MOD_GPT2, MOD_QWEN, MOD_TUNED, MOD_DECODE, MOD_PREFILL, MOD_PROBE, NMOD };
 static const struct {
     const char *name;
     const unsigned char *start, *end;
@@ -41,6 +42,7 @@ static const struct {
     {"qwen_kernels", sgpu_co_qwen_kernels, sgpu_co_qwen_kernels_end},
     {"sgpu_tuned", sgpu_co_sgpu_tuned, sgpu_co_sgpu_tuned_end},
     {"sgpu_decode", sgpu_co_sgpu_decode, sgpu_co_sgpu_decode_end},
+    {"sgpu_prefill", sgpu_co_sgpu_prefill, sgpu_co_sgpu_prefill_end},
     {"sgpu_probe", sgpu_co_sgpu_probe, sgpu_co_sgpu_probe_end},
 };
 
@@ -95,6 +97,13 @@ static const char *g_dec_fam[NDECFAM] = {"qkv", "gateup", "res", "lmhead", "g2qk
 static int dec_is_pair(int f) { return f == DEC_QKV || f == DEC_GATEUP; }
 static int dec_vec(int f) { return f >= DEC_G2QKV ? 4 : 8; }
 
+/* Prompt products in fp16 pieces (sgpu_prefill.hip): tokens / 64 and weight rows / 64 of a
+ * block's tile, and the blocks that a CU holds (registers, LDS). */
+static const struct {
+    int tf, nf, per_cu;
+} g_pf_mm[] = {{2, 4, 2}, {2, 2, 2}, {1, 2, 4}, {1, 1, 5}};
+#define NPFMM 4
+
 typedef struct {
     int ready;
     int cus;
@@ -105,6 +114,7 @@ typedef struct {
     hipFunction_t dec_attn[3], dec_embed, dec_argmax_part, dec_argmax_embed;
     hipFunction_t dec_g2embed, dec_argmax_g2embed;
     hipFunction_t pf_embed, pf_gemm, pf_qkv_post, pf_attn[3], pf_swiglu;
+    hipFunction_t pf_mm[NPFMM], pf_gateup[2], pf_rms, h16_flush;
     /* Split-K workspaces, one per stream that has launched split work (slot 0: the null
      * stream, made with the device state): partial tiles (SK_WS_FLOATS) and arrival counters
      * (SK_MAX_TILES, zero between launches).  Launches on one stream run in order, so a
@@ -212,7 +222,7 @@ static int load_device(int dev) {
         const char *pattn[3] = {"sgpu_pf_attn32", "sgpu_pf_attn64", "sgpu_pf_attn128"};
         for (int j = 0; j < 3; j++)
             if (hipModuleGetFunction(&d->dec_attn[j], d->mod[MOD_DECODE], attn[j]) != hipSuccess ||
-                hipModuleGetFunction(&d->pf_attn[j], d->mod[MOD_DECODE], pattn[j]) != hipSuccess) {
+                hipModuleGetFunction(&d->pf_attn[j], d->mod[MOD_PREFILL], pattn[j]) != hipSuccess) {
                 rc = SGPU_ERR_NO_KERNEL;
                 goto fail;
             }
@@ -224,9 +234,21 @@ static int load_device(int dev) {
             hipModuleGetFunction(&d->pf_embed, d->mod[MOD_DECODE], "sgpu_pf_embed") != hipSuccess ||
             hipModuleGetFunction(&d->pf_gemm, d->mod[MOD_DECODE], "sgpu_pf_gemm") != hipSuccess ||
             hipModuleGetFunction(&d->pf_qkv_post, d->mod[MOD_DECODE], "sgpu_pf_qkv_post") != hipSuccess ||
-            hipModuleGetFunction(&d->pf_swiglu, d->mod[MOD_DECODE], "sgpu_pf_swiglu") != hipSuccess) {
+            hipModuleGetFunction(&d->pf_swiglu, d->mod[MOD_DECODE], "sgpu_pf_swiglu") != hipSuccess ||
+            hipModuleGetFunction(&d->pf_gateup[0], d->mod[MOD_PREFILL], "sgpu_pf_gateup_1") != hipSuccess ||
+            hipModuleGetFunction(&d->pf_gateup[1], d->mod[MOD_PREFILL], "sgpu_pf_gateup_2") != hipSuccess ||
+            hipModuleGetFunction(&d->pf_rms, d->mod[MOD_PREFILL], "sgpu_pf_rms") != hipSuccess ||
+            hipModuleGetFunction(&d->h16_flush, d->mod[MOD_PREFILL], "sgpu_h16_flush") != hipSuccess) {
             rc = SGPU_ERR_NO_KERNEL;
             goto fail;
+        }
+        for (int j = 0; j < NPFMM; j++) {
+            char name[64];
+            snprintf(name, sizeof name, "sgpu_pf_mm_%d%d", g_pf_mm[j].tf, g_pf_mm[j].nf);
+            if (hipModuleGetFunction(&d->pf_mm[j], d->mod[MOD_PREFILL], name) != hipSuccess) {
+                rc = SGPU_ERR_NO_KERNEL;
+                goto fail;
+            }
         }
     }
     /* the null stream's split-K workspace, counters zeroed once (every launch leaves them at zero) */
@@ -1616,10 +1638,10 @@ int sgpu_internal_pf_qkv_post(float *qkv, int T, int pos0, const float *cosT, co
     return launch(d->pf_qkv_post, g, b, stream, args);
 }
 
-int sgpu_internal_pf_attn(const float *qkv, const float *kc, const float *vc, float *out, int T, int pos0, int NH,
-                          int NKV, int HD, float scale, void *stream) {
+int sgpu_internal_pf_attn(const float *qkv, const float *kc, const float *vc, float *out, uint16_t *P, float *pd,
+                          int T, int pos0, int NH, int NKV, int HD, float scale, void *stream) {
     const int j = HD == 32 ? 0 : HD == 64 ? 1 : HD == 128 ? 2 : -1;
-    if (j < 0 || !qkv || !kc || !vc || !out || T <= 0 || T > 65535 || pos0 < 0 || pos0 + T > 8192 || NKV <= 0 ||
+    if (j < 0 || !qkv || !kc || !vc || !(P ? pd != NULL && HD >= 64 : out != NULL) || T <= 0 || T > 65535 || pos0 < 0 || pos0 + T > 8192 || NKV <= 0 ||
         NH <= 0 || NH % NKV)
         return SGPU_ERR_INVALID_ARG;
     int rc;
@@ -1627,7 +1649,8 @@ int sgpu_internal_pf_attn(const float *qkv, const float *kc, const float *vc, fl
     if (!d) return rc;
     int QKVD = (NH + 2 * NKV) * HD;
     unsigned g[3] = {(unsigned)NH * cdiv(T, 32), 1, 1}, b[3] = {256, 1, 1};   /* a block per head and 32 rows */
-    void *args[] = {(void *)&qkv, (void *)&kc, (void *)&vc, (void *)&out, &pos0, &T, &NH, &NKV, &scale, &QKVD};
+    void *args[] = {(void *)&qkv, (void *)&kc, (void *)&vc, (void *)&out, (void *)&P, (void *)&pd,
+                    &pos0, &T, &NH, &NKV, &scale, &QKVD};
     return launch(d->pf_attn[j], g, b, stream, args);
 }
 
@@ -1639,6 +1662,87 @@ int sgpu_internal_pf_swiglu(const float *Y, float *G, int FC, int T, void *strea
     unsigned g[3] = {(unsigned)elem_grid((int)umin((unsigned)((long long)T * FC), 0x7fffffffu)), 1, 1}, b[3] = {256, 1, 1};
     void *args[] = {(void *)&Y, (void *)&G, &FC, &T};
     return launch(d->pf_swiglu, g, b, stream, args);
+}
+
+/* ---- prompt products in fp16 pieces (sgpu_prefill.hip) ---- */
+int sgpu_internal_h16_flush(uint16_t *w, size_t n, void *stream) {
+    if (!w || n == 0 || n % 8 || ((uintptr_t)w & 15)) return SGPU_ERR_INVALID_ARG;
+    int rc;
+    devstate *d = cur(&rc);
+    if (!d) return rc;
+    const size_t blocks = (n / 8 + 255) / 256;
+    unsigned g[3] = {(unsigned)(blocks < 8192 ? blocks : 8192), 1, 1}, b[3] = {256, 1, 1};
+    void *args[] = {(void *)&w, &n};
+    return launch(d->h16_flush, g, b, stream, args);
+}
+
+int sgpu_internal_pf_rms(const float *x, const uint16_t *w, uint16_t *P, float *pd, int n, float eps, int rows,
+                         void *stream) {
+    if (!x || !w || !P || !pd || n <= 0 || n % 64 || rows <= 0) return SGPU_ERR_INVALID_ARG;
+    int rc;
+    devstate *d = cur(&rc);
+    if (!d) return rc;
+    unsigned g[3] = {(unsigned)rows, 1, 1}, b[3] = {256, 1, 1};
+    void *args[] = {(void *)&x, (void *)&w, (void *)&P, (void *)&pd, &n, &eps};
+    return launch(d->pf_rms, g, b, stream, args);
+}
+
+/* Estimated cycles of a product on tile shape j with K split S ways: rounds of blocks over the
+ * CUs, each step costing the matrix work of the blocks that share a CU or, when that is less, one
+ * block's own work after its loads have arrived. */
+#define PF_LOAD_CYCLES 2500
+static double pf_mm_cost(int j, long long tiles, int ng, int S, int cus) {
+    const double m = 384.0 * g_pf_mm[j].tf * g_pf_mm[j].nf;
+    const int per = g_pf_mm[j].per_cu, steps = (ng + S - 1) / S;
+    const long long slots = (long long)cus * per, units = tiles * S, full = units / slots, rem = units % slots;
+    const long long last = (rem + cus - 1) / cus;
+    double c = 0;
+    if (full) c += (double)full * (per * m > m + PF_LOAD_CYCLES ? per * m : m + PF_LOAD_CYCLES);
+    if (last) c += last * m > m + PF_LOAD_CYCLES ? last * m : m + PF_LOAD_CYCLES;
+    return c * steps + (S > 1 ? 3000.0 + 60.0 * S * g_pf_mm[j].tf * g_pf_mm[j].nf : 0.0);
+}
+
+int sgpu_internal_pf_mm(const uint16_t *W, const uint16_t *X, const float *xd, const float *bias, float *Y, int K,
+                        int N, int T, float *ws, unsigned *cnt, int accum, void *stream) {
+    if (!W || !X || !xd || !Y || K <= 0 || N <= 0 || T <= 0 || K % 64 || N % 64 || (long long)N * K >= 1LL << 30 ||
+        3LL * T * K >= 1LL << 30)
+        return SGPU_ERR_INVALID_ARG;
+    int rc;
+    devstate *d = cur(&rc);
+    if (!d) return rc;
+    int best = 0, S = 1;
+    double least = 0;
+    for (int j = 0; j < NPFMM; j++) {
+        const long long tiles = (long long)cdiv(T, 64 * g_pf_mm[j].tf) * cdiv(N, 64 * g_pf_mm[j].nf);
+        const int rec = 4096 * g_pf_mm[j].tf * g_pf_mm[j].nf;
+        for (int s = 1; s <= 16 && s <= K / 64; s++) {
+            if (s > 1 && (!ws || !cnt || tiles > (long long)SGPU_NT_CNT || s * tiles * rec > (long long)SGPU_PF_WS_FLOATS))
+                break;
+            const double c = pf_mm_cost(j, tiles, K / 64, s, d->cus);
+            if (least == 0 || c < least) least = c, best = j, S = s;
+        }
+    }
+    const long long units = (long long)cdiv(T, 64 * g_pf_mm[best].tf) * cdiv(N, 64 * g_pf_mm[best].nf) * S;
+    unsigned g[3] = {(unsigned)units, 1, 1}, b[3] = {256, 1, 1};
+    void *args[] = {(void *)&W, (void *)&X, (void *)&xd, (void *)&bias, (void *)&Y, &K, &N, &T, &S,
+                    (void *)&ws, (void *)&cnt, &accum};
+    return launch(d->pf_mm[best], g, b, stream, args);
+}
+
+int sgpu_internal_pf_gateup(const uint16_t *W, const uint16_t *X, const float *xd, uint16_t *P, float *pd, int K,
+                            int FC, int T, void *stream) {
+    if (!W || !X || !xd || !P || !pd || K <= 0 || FC <= 0 || T <= 0 || K % 64 || FC % 64 ||
+        2LL * FC * K >= 1LL << 30 || 3LL * T * K >= 1LL << 30)
+        return SGPU_ERR_INVALID_ARG;
+    int rc;
+    devstate *d = cur(&rc);
+    if (!d) return rc;
+    /* 128 tokens a block, or 64 where that fills the last round better */
+    const long long cols = cdiv(FC, 128), t2 = cdiv(T, 128) * cols, t1 = cdiv(T, 64) * cols;
+    const int two = pf_mm_cost(0, t2, K / 64, 1, d->cus) <= pf_mm_cost(0, (t1 + 1) / 2, K / 64, 1, d->cus);
+    unsigned g[3] = {(unsigned)(two ? t2 : t1), 1, 1}, b[3] = {256, 1, 1};
+    void *args[] = {(void *)&W, (void *)&X, (void *)&xd, (void *)&P, (void *)&pd, &K, &FC, &T};
+    return launch(d->pf_gateup[two], g, b, stream, args);
 }
 
 /* ---- GPT-2 fused decode (sgpu_decode.hip, fp32 weights) ---- */

@@ -350,165 +350,6 @@ __device__ __forceinline__ void amax_block256(float& bv, int& bi, float* sv, int
     for (int i = 1; i < 4; i++) amax_merge(bv, bi, sv[i], si[i]);
 }
 
-// Causal attention for prompt rows on the fp32 matrix cores: T query rows at positions pos0..
-// (row t's q rotated in place in its qkv vector of length QKVD) over cached positions
-// 0..pos0+t, one block per query head and 32 query rows, output row t of out (NH*HD floats).
-//
-// Bound: the matrix cores (4*HD flop per query, key and head).  The keys are taken in tiles of
-// 32, dealt to the block's four waves (wave w: tiles w, w+4, ..); each wave keeps its own
-// running maximum, sum and output over its tiles (online softmax) and the four are merged once
-// through LDS at the end, so the key loop has no barrier and a short prompt still fills the
-// CUs' SIMDs.  Both products are laid out so that no operand passes through LDS:
-//  * scores transposed, S^T = K Q^T: lane (l32, h) feeds key l32's dims HD/2*h.. as A and query
-//    l32's as B (16-byte loads; the k order of a dot product is free), so accumulator r of a
-//    lane is key 8*(r/4) + 4*h + r%4 of query l32 and the softmax over keys is in-lane, plus
-//    one exchange between the lane halves;
-//  * O^T = V^T P^T: step r multiplies the keys the lanes hold in accumulator r, so P is the B
-//    operand where it lies, and A is V[that key][NB*l32 + j] for dim block j (NB = HD/32
-//    consecutive dims per lane: one 4*NB-byte load per step).
-// K and V of the wave's next tile are loaded while this tile's softmax and second product run.
-// Loads go through buffer resources that end at the last valid key row: rows past it read as
-// zero and are masked.  The heavy blocks (last rows) are dispatched first.
-// Measured against one block per head and row on the vector ALUs, which read K and V once per
-// row: 50 -> 17 us a launch at 500 rows, 14 query and 2 KV heads of 64 (the whole prompt 6.89 ->
-// 6.08 ms); a 3001-row prompt in chunks of 512 rows 232 -> 41 us a launch on average (67.1 ->
-// 39.5 ms).
-template <int HD>
-__device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const float* __restrict__ kc,
-                                        const float* __restrict__ vc, float* __restrict__ out, int pos0, int T, int NH,
-                                        int NKV, float scale, int QKVD) {
-    typedef float f32x16 __attribute__((ext_vector_type(16)));
-    constexpr int HH = HD / 2, NB = HD / 32, P = HD + 1;
-    typedef uint32_t vseg __attribute__((ext_vector_type(NB)));
-    __shared__ float part[4][32][P];
-    __shared__ float ml[4][2][32];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int l32 = lane & 31, h = lane >> 5;
-    const int head = blockIdx.x % NH, q0 = ((T + 31) / 32 - 1 - blockIdx.x / NH) * 32;
-    const int KVD = NKV * HD, g = head / (NH / NKV);
-    const int n = pos0 + min(T, q0 + 32);             // keys that some row of the block reads
-    const int ntile = (n + 31) / 32, qpos = pos0 + q0 + l32;
-
-    float qv[HH];
-    {
-        const float* qr = qkv + (size_t)min(q0 + l32, T - 1) * QKVD + (size_t)head * HD + HH * h;
-#pragma unroll
-        for (int v = 0; v < HH / 4; v++) {
-            const sgpu_f32x4 a = *reinterpret_cast<const sgpu_f32x4*>(qr + 4 * v);
-#pragma unroll
-            for (int e = 0; e < 4; e++) qv[4 * v + e] = a[e];
-        }
-    }
-    sgpu_f32x4 kr[HH / 4];
-    vseg vr[16];
-    const int koff = (l32 * KVD + HH * h) * 4, voff = (4 * h * KVD + NB * l32) * 4;
-    auto tile_rsrc = [&](const float* c, int t) __attribute__((always_inline)) {
-        const int rows = max(n - 32 * t, 0);
-        return __builtin_amdgcn_make_buffer_rsrc((void*)(c + (size_t)g * HD + (size_t)t * 32 * KVD), (short)0,
-                                                 rows > 0 ? (min(rows, 32) * KVD - (KVD - HD)) * 4 : 0, 0x00020000);
-    };
-    auto load_k = [&](int t) __attribute__((always_inline)) {
-        const __amdgpu_buffer_rsrc_t rs = tile_rsrc(kc, t);
-#pragma unroll
-        for (int v = 0; v < HH / 4; v++)
-            kr[v] = __builtin_bit_cast(sgpu_f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, koff + 16 * v, 0, 0));
-    };
-    auto load_v = [&](int t) __attribute__((always_inline)) {
-        const __amdgpu_buffer_rsrc_t rs = tile_rsrc(vc, t);
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int o = voff + (8 * (r / 4) + r % 4) * KVD * 4;
-            if constexpr (NB == 1) vr[r][0] = __builtin_amdgcn_raw_buffer_load_b32(rs, o, 0, 0);
-            else if constexpr (NB == 2) vr[r] = __builtin_bit_cast(vseg, __builtin_amdgcn_raw_buffer_load_b64(rs, o, 0, 0));
-            else vr[r] = __builtin_bit_cast(vseg, __builtin_amdgcn_raw_buffer_load_b128(rs, o, 0, 0));
-        }
-    };
-
-    f32x16 o[NB];
-#pragma unroll
-    for (int j = 0; j < NB; j++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) o[j][r] = 0.0f;
-    float m = -INFINITY, l = 0.0f;
-    load_k(wave);
-    load_v(wave);
-    for (int t = wave; t < ntile; t += 4) {
-        f32x16 s, s1;
-#pragma unroll
-        for (int r = 0; r < 16; r++) s[r] = s1[r] = 0.0f;
-#pragma unroll
-        for (int k = 0; k < HH; k += 2) {             // two accumulators: no MFMA waits for the one before it
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[k / 4][k % 4], qv[k], s, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[k / 4][k % 4 + 1], qv[k + 1], s1, 0, 0, 0);
-        }
-        load_k(t + 4);
-        float mx = -INFINITY;
-#pragma unroll
-        for (int r = 0; r < 16; r++) s[r] = (s[r] + s1[r]) * scale;
-        if (32 * t + 31 > pos0 + q0) {                // the tile reaches past some row's own position
-#pragma unroll
-            for (int r = 0; r < 16; r++)
-                if (32 * t + 8 * (r / 4) + 4 * h + r % 4 > qpos) s[r] = -INFINITY;
-        }
-#pragma unroll
-        for (int r = 0; r < 16; r++) mx = fmaxf(mx, s[r]);
-        mx = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32)));
-        const float base = mx == -INFINITY ? 0.0f : mx;   // every key so far masked: weights are all zero
-        const float al = expf(m - base);
-        m = mx;
-        float sum = 0.0f;
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            s[r] = expf(s[r] - base);
-            sum += s[r];
-        }
-        l = l * al + sum;
-        if (__any(al != 1.0f)) {
-#pragma unroll
-            for (int j = 0; j < NB; j++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) o[j][r] *= al;
-        }
-#pragma unroll
-        for (int r = 0; r < 16; r++)
-#pragma unroll
-            for (int j = 0; j < NB; j++)
-                o[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(vr[r][j]), s[r], o[j], 0, 0, 0);
-        load_v(t + 4);
-    }
-    l += __shfl_xor(l, 32);
-    if (h == 0) {
-        ml[wave][0][l32] = m;
-        ml[wave][1][l32] = l;
-    }
-#pragma unroll
-    for (int j = 0; j < NB; j++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) part[wave][l32][NB * (8 * (r / 4) + 4 * h + r % 4) + j] = o[j][r];
-    __syncthreads();
-    // Merge: 8 threads per query row, HD/8 dims each; the four waves in order.
-    const int q = threadIdx.x / 8, d0 = (threadIdx.x % 8) * (HD / 8);
-    if (q0 + q >= T) return;
-    float M = ml[0][0][q];
-#pragma unroll
-    for (int w = 1; w < 4; w++) M = fmaxf(M, ml[w][0][q]);
-    if (M == -INFINITY) M = 0.0f;
-    float wt[4], L = 0.0f;
-#pragma unroll
-    for (int w = 0; w < 4; w++) {
-        wt[w] = expf(ml[w][0][q] - M);
-        L = __builtin_fmaf(ml[w][1][q], wt[w], L);
-    }
-    float* orow = out + (size_t)(q0 + q) * NH * HD + (size_t)head * HD + d0;
-#pragma unroll
-    for (int e = 0; e < HD / 8; e++) {
-        float v = 0.0f;
-#pragma unroll
-        for (int w = 0; w < 4; w++) v = __builtin_fmaf(part[w][q][d0 + e], wt[w], v);
-        orow[e] = v / L;
-    }
-}
-
 }  // namespace
 
 using sgpu::WF16;
@@ -658,22 +499,6 @@ __global__ void sgpu_pf_qkv_post(float* __restrict__ qkv, int T, int pos0, const
             vc[(size_t)pos * KVD + j] = row[(NH + NKV) * HD + j];
         }
     }
-}
-
-__global__ void __launch_bounds__(256) sgpu_pf_attn64(const float* __restrict__ qkv, const float* __restrict__ kc,
-                                                      const float* __restrict__ vc, float* __restrict__ out, int pos0,
-                                                      int T, int NH, int NKV, float scale, int QKVD) {
-    pf_attn<64>(qkv, kc, vc, out, pos0, T, NH, NKV, scale, QKVD);
-}
-__global__ void __launch_bounds__(256) sgpu_pf_attn32(const float* __restrict__ qkv, const float* __restrict__ kc,
-                                                      const float* __restrict__ vc, float* __restrict__ out, int pos0,
-                                                      int T, int NH, int NKV, float scale, int QKVD) {
-    pf_attn<32>(qkv, kc, vc, out, pos0, T, NH, NKV, scale, QKVD);
-}
-__global__ void __launch_bounds__(256) sgpu_pf_attn128(const float* __restrict__ qkv, const float* __restrict__ kc,
-                                                       const float* __restrict__ vc, float* __restrict__ out, int pos0,
-                                                       int T, int NH, int NKV, float scale, int QKVD) {
-    pf_attn<128>(qkv, kc, vc, out, pos0, T, NH, NKV, scale, QKVD);
 }
 
 // G[t][i] = silu(Y[t][i]) * Y[t][FC + i] for gate|up rows of 2*FC (the swiglu kernel's

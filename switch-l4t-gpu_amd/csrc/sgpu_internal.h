@@ -62,9 +62,23 @@ SGPU_HIDDEN int sgpu_internal_gemv_multi(const float *W, const float *X, const f
 #define SGPU_NT_CNT 1024u
 SGPU_HIDDEN int sgpu_internal_pf_qkv_post(float *qkv, int T, int pos0, const float *cosT, const float *sinT,
                                           float *kc, float *vc, int NH, int NKV, int HD, void *stream);
-SGPU_HIDDEN int sgpu_internal_pf_attn(const float *qkv, const float *kc, const float *vc, float *out, int T,
-                                      int pos0, int NH, int NKV, int HD, float scale, void *stream);
+/* Output rows to out, or (P != NULL, HD >= 64) as fp16 pieces to P with their scales in pd. */
+SGPU_HIDDEN int sgpu_internal_pf_attn(const float *qkv, const float *kc, const float *vc, float *out, uint16_t *P,
+                                      float *pd, int T, int pos0, int NH, int NKV, int HD, float scale, void *stream);
 SGPU_HIDDEN int sgpu_internal_pf_swiglu(const float *Y, float *G, int FC, int T, void *stream);
+/* The prompt's products on the fp16 matrix cores (sgpu_prefill.hip).  x rows are held as three
+ * fp16 pieces (P: 3*K codes a row) with one scale per 64 values (pd: K/64 floats a row); weights
+ * have their subnormal codes cleared (h16_flush, once).  pf_mm: Y[T][N] = X W^T + bias, added to
+ * Y if accum != 0; K split over blocks through ws (SGPU_PF_WS_FLOATS floats) and cnt
+ * (SGPU_NT_CNT counters, kept at zero).  pf_gateup: SwiGLU of gate|up rows of 2*FC, as pieces. */
+#define SGPU_PF_WS_FLOATS (8u << 20)
+SGPU_HIDDEN int sgpu_internal_h16_flush(uint16_t *w, size_t n, void *stream);
+SGPU_HIDDEN int sgpu_internal_pf_rms(const float *x, const uint16_t *w, uint16_t *P, float *pd, int n, float eps,
+                                     int rows, void *stream);
+SGPU_HIDDEN int sgpu_internal_pf_mm(const uint16_t *W, const uint16_t *X, const float *xd, const float *bias,
+                                    float *Y, int K, int N, int T, float *ws, unsigned *cnt, int accum, void *stream);
+SGPU_HIDDEN int sgpu_internal_pf_gateup(const uint16_t *W, const uint16_t *X, const float *xd, uint16_t *P,
+                                        float *pd, int K, int FC, int T, void *stream);
 /* GPT-2 fused decode (fp32 weights), see gpt2.c. */
 SGPU_HIDDEN int sgpu_internal_g2_qkv(const float *W, int K, int N, const float *x, const float *lnw,
                                      const float *lnb, float eps, const float *bias, float *q, float *kc,

@@ -263,6 +263,46 @@ def test_engine_prefill_attention_tiles(gpu, og, heads, T):
     fresh.close()
 
 
+# The prompt products in fp16 pieces (from 65 rows on, 64-wide heads and whole 64-blocks): token
+# tiles of 64 and 128, column tiles of 64 to 256 and their remainders.
+@pytest.mark.parametrize("T", [65, 128, 129, 250])
+@pytest.mark.parametrize("sizes", [(3, 1, 64, 192), (14, 2, 64, 704), (4, 2, 128, 1024)], ids=["c192", "c896", "hd128"])
+def test_engine_prefill_pieces_tiles(gpu, og, sizes, T):
+    NH, NKV, HD, FC = sizes
+    test_engine_prefill_matches_golden(gpu, og, dict(
+        cfg=dict(V=300, C=NH * HD, NL=2, NH=NH, NKV=NKV, HD=HD, FC=FC, CTX=260), T=T))
+
+
+def test_engine_prefill_pieces_weight_codes(gpu, og):
+    """Layer weights with subnormal codes (read as 0) and codes of exponent 31 (finite values in
+    the reference), in a gate row, an up row and the o and down matrices; and a prompt longer
+    than one whose buffers the engine holds already."""
+    cfg = dict(V=300, C=128, NL=2, NH=2, NKV=1, HD=64, FC=192, CTX=700)
+    C, FC, Q = 128, 192, 256
+    blob = np.array(gpu.qwen_random_blob(gpu.qwen_cfg(**cfg), seed=53, std=0.05), copy=True).view(np.uint8)
+    l0 = cfg["V"] * C * 2 + 2 * cfg["CTX"] * 32 * 4
+    layer = (C + Q * C + Q + C * C + C + 2 * FC * C + C * FC)
+    h = blob[l0:l0 + 2 * layer * cfg["NL"]].view(np.uint16)
+    rng = np.random.default_rng(5)
+    o = C + Q * C + Q
+    gateup = o + C * C + C
+    down = gateup + 2 * FC * C
+    for start, n in ((C, Q * C), (o, C * C), (gateup, 2 * FC * C), (down, C * FC)):
+        at = start + rng.integers(0, n, 40)
+        h[at] = rng.integers(1, 0x400, 40) | (rng.integers(0, 2, 40) << 15)
+    for at in (gateup + 5 * C + 3, gateup + (FC + 70) * C + 9, o + 17 * C + 1, down + 3 * FC + 100):
+        h[at] = 0x7c01
+    ids = [int(v) for v in rng.integers(0, cfg["V"], 600)]
+    eng = gpu.QwenEngine(gpu.qwen_cfg(**cfg), blob, PATHS["fused"])
+    for T in (100, 600):
+        gold = og.QwenGolden(og.qwen_cfg(**cfg), blob, NT)
+        for p in range(T):
+            want = gold.forward(ids[p], p, p == T - 1)
+        got = eng.prefill(ids[:T])
+        assert np.isfinite(want).all() and np.abs(got - want).max() <= 1e-4 * np.abs(want).max()
+    eng.close()
+
+
 def test_engine_prefill_rejects_bad_ids(gpu):
     cfg = SMALL
     eng = gpu.QwenEngine(gpu.qwen_cfg(**cfg), gpu.qwen_random_blob(gpu.qwen_cfg(**cfg), seed=3), PATHS["fused"])
