@@ -98,11 +98,13 @@ static int dec_is_pair(int f) { return f == DEC_QKV || f == DEC_GATEUP; }
 static int dec_vec(int f) { return f >= DEC_G2QKV ? 4 : 8; }
 
 /* Prompt products in fp16 pieces (sgpu_prefill.hip): tokens / 64 and weight rows / 64 of a
- * block's tile, and the blocks that a CU holds (registers, LDS). */
+ * block's tile, and the rule's us per step of 64 k: of a CU's first block, and of each block
+ * when several share a CU. */
 static const struct {
-    int tf, nf, per_cu;
-} g_pf_mm[] = {{2, 4, 2}, {2, 2, 2}, {1, 2, 4}, {1, 1, 5}};
-#define NPFMM 4
+    int tf, nf;
+    double first, each;
+} g_pf_mm[] = {{2, 2, 4.6, 2.25}, {1, 2, 2.2, 1.18}, {1, 1, 1.3, 0.77}};
+#define NPFMM 3
 
 typedef struct {
     int ready;
@@ -114,7 +116,7 @@ typedef struct {
     hipFunction_t dec_attn[3], dec_embed, dec_argmax_part, dec_argmax_embed;
     hipFunction_t dec_g2embed, dec_argmax_g2embed;
     hipFunction_t pf_embed, pf_gemm, pf_qkv_post, pf_attn[3], pf_swiglu;
-    hipFunction_t pf_mm[NPFMM], pf_gateup[2], pf_rms, h16_flush;
+    hipFunction_t pf_mm[NPFMM], pf_gateup, pf_rms, h16_flush;
     /* Split-K workspaces, one per stream that has launched split work (slot 0: the null
      * stream, made with the device state): partial tiles (SK_WS_FLOATS) and arrival counters
      * (SK_MAX_TILES, zero between launches).  Launches on one stream run in order, so a
@@ -235,8 +237,7 @@ static int load_device(int dev) {
             hipModuleGetFunction(&d->pf_gemm, d->mod[MOD_DECODE], "sgpu_pf_gemm") != hipSuccess ||
             hipModuleGetFunction(&d->pf_qkv_post, d->mod[MOD_DECODE], "sgpu_pf_qkv_post") != hipSuccess ||
             hipModuleGetFunction(&d->pf_swiglu, d->mod[MOD_DECODE], "sgpu_pf_swiglu") != hipSuccess ||
-            hipModuleGetFunction(&d->pf_gateup[0], d->mod[MOD_PREFILL], "sgpu_pf_gateup_1") != hipSuccess ||
-            hipModuleGetFunction(&d->pf_gateup[1], d->mod[MOD_PREFILL], "sgpu_pf_gateup_2") != hipSuccess ||
+            hipModuleGetFunction(&d->pf_gateup, d->mod[MOD_PREFILL], "sgpu_pf_gateup") != hipSuccess ||
             hipModuleGetFunction(&d->pf_rms, d->mod[MOD_PREFILL], "sgpu_pf_rms") != hipSuccess ||
             hipModuleGetFunction(&d->h16_flush, d->mod[MOD_PREFILL], "sgpu_h16_flush") != hipSuccess) {
             rc = SGPU_ERR_NO_KERNEL;
@@ -1687,19 +1688,14 @@ int sgpu_internal_pf_rms(const float *x, const uint16_t *w, uint16_t *P, float *
     return launch(d->pf_rms, g, b, stream, args);
 }
 
-/* Estimated cycles of a product on tile shape j with K split S ways: rounds of blocks over the
- * CUs, each step costing the matrix work of the blocks that share a CU or, when that is less, one
- * block's own work after its loads have arrived. */
-#define PF_LOAD_CYCLES 2500
+/* Estimated us of a product on tile shape j with K split S ways: the steps of the fullest CU,
+ * and with a split the partial tiles' way through memory.  The figures are fitted to timings of
+ * every shape and split at 66 to 3001 rows (N 1152, K 896; 896, 896; 896, 4864): the choice is
+ * the fastest or within 14% of it (21% at 66 rows, K 896). */
 static double pf_mm_cost(int j, long long tiles, int ng, int S, int cus) {
-    const double m = 384.0 * g_pf_mm[j].tf * g_pf_mm[j].nf;
-    const int per = g_pf_mm[j].per_cu, steps = (ng + S - 1) / S;
-    const long long slots = (long long)cus * per, units = tiles * S, full = units / slots, rem = units % slots;
-    const long long last = (rem + cus - 1) / cus;
-    double c = 0;
-    if (full) c += (double)full * (per * m > m + PF_LOAD_CYCLES ? per * m : m + PF_LOAD_CYCLES);
-    if (last) c += last * m > m + PF_LOAD_CYCLES ? last * m : m + PF_LOAD_CYCLES;
-    return c * steps + (S > 1 ? 3000.0 + 60.0 * S * g_pf_mm[j].tf * g_pf_mm[j].nf : 0.0);
+    const long long u = (tiles * S + cus - 1) / cus;
+    const double step = u * g_pf_mm[j].each > g_pf_mm[j].first ? u * g_pf_mm[j].each : g_pf_mm[j].first;
+    return (ng + S - 1) / S * step + (S > 1 ? 1.6 + 4.9 * g_pf_mm[j].tf * g_pf_mm[j].nf * (double)u : 0.0);
 }
 
 int sgpu_internal_pf_mm(const uint16_t *W, const uint16_t *X, const float *xd, const float *bias, float *Y, int K,
@@ -1737,12 +1733,9 @@ int sgpu_internal_pf_gateup(const uint16_t *W, const uint16_t *X, const float *x
     int rc;
     devstate *d = cur(&rc);
     if (!d) return rc;
-    /* 128 tokens a block, or 64 where that fills the last round better */
-    const long long cols = cdiv(FC, 128), t2 = cdiv(T, 128) * cols, t1 = cdiv(T, 64) * cols;
-    const int two = pf_mm_cost(0, t2, K / 64, 1, d->cus) <= pf_mm_cost(0, (t1 + 1) / 2, K / 64, 1, d->cus);
-    unsigned g[3] = {(unsigned)(two ? t2 : t1), 1, 1}, b[3] = {256, 1, 1};
+    unsigned g[3] = {cdiv(T, 64) * cdiv(FC, 128), 1, 1}, b[3] = {256, 1, 1};
     void *args[] = {(void *)&W, (void *)&X, (void *)&xd, (void *)&P, (void *)&pd, &K, &FC, &T};
-    return launch(d->pf_gateup[two], g, b, stream, args);
+    return launch(d->pf_gateup, g, b, stream, args);
 }
 
 /* ---- GPT-2 fused decode (sgpu_decode.hip, fp32 weights) ---- */

@@ -14,9 +14,8 @@
 // chosen over the finite ones.
 //
 // Measured against the same layers on fp32 MFMA tiles (sgpu_pf_gemm, 32x32 per block): a prompt
-// of 500 rows of the Qwen2.5-0.5B sizes 6.08 -> 4.52 ms, of 3001 rows 39.5 -> 13.5 ms; distance
-// of the logits from a 64-bit forward 9.7e-7 -> 6.9e-7 and 9.2e-7 -> 9.7e-7 (1.1e-6 at the same
-// inputs).
+// of 500 rows of the Qwen2.5-0.5B sizes 6.08 -> 3.35 ms, of 3001 rows 39.5 -> 12.1 ms; distance
+// of the logits from a 64-bit forward 1.1e-6 -> 6.4e-7 and 9.3e-7 -> 8.0e-7.
 //
 // This code object keeps fp16 subnormals (the pieces use them).  The reference reads subnormal
 // weights as +0: the engine clears those codes once, where it uploads the weights
@@ -76,12 +75,14 @@ enum { EPI_STORE, EPI_SWIGLU };
 // Y[t][n] = X[t] . W[n] + bias?[n] (EPI_STORE; accum != 0: added to Y), or silu(gate) * up as
 // pieces for the next product (EPI_SWIGLU: W holds N gate rows, then N up rows).
 //
-// Bound: the matrix cores.  A block of 2x2 waves computes 64*TF tokens x 64*NF weight rows, a
-// wave 32*TF x 32*NF of them.  Per step of 64 k the block's pieces and weights go straight into
-// LDS (16 bytes a lane, no registers; a row's eight 16-byte chunks are stored at chunk ^ (row %
-// 8), so that the operand reads of eight consecutive rows use all banks); there is one buffer,
+// Bound: the matrix cores, and below some 1000 rows the steps' loads.  (These cores reach 1.7-2.0
+// PFLOP/s on dense operands, 2.5 on zeros; gate|up at 3001 rows runs at 1.04 PFLOP/s of piece
+// products, 1.4 with its loads taken out.)  A block of 2x2 waves computes 64*TF tokens x 64*NF weight rows, a
+// wave 32*TF x 32*NF of them in 16x16 tiles.  Per step of 64 k the block's pieces and weights go straight into
+// LDS (16 bytes a lane, no registers; a row's eight 16-byte chunks are stored at chunk ^ (row / 2
+// % 8), so that the operand reads of sixteen consecutive rows use all banks); there is one buffer,
 // and the two or more blocks on a CU cover each other's loads.  The products run transposed
-// (weights as A), so a lane holds one token per 32x32 tile and scales its step's sum with one
+// (weights as A), so a lane holds one token per 16x16 tile and scales its step's sum with one
 // factor; four consecutive n per lane make 16-byte stores.  Within a step the smallest pieces
 // are summed first.
 // S > 1: K split over S blocks per tile by the hand-off of sgpu_device.h; ws holds S * tiles
@@ -95,25 +96,28 @@ __device__ __forceinline__ void pf_mm(const uint16_t* __restrict__ W, const uint
                                       int N, int T, int S, float* __restrict__ ws, unsigned* __restrict__ cnt,
                                       int accum) {
     constexpr int TT = 64 * TF, NR = 64 * NF;              // tokens and weight rows per block
+    constexpr int TM = 2 * TF, NM = 2 * NF;                // a wave's 16x16 tiles
     constexpr int NC = EPI == EPI_SWIGLU ? NR / 2 : NR;    // output columns per block
     static_assert(EPI == EPI_STORE || NF == 4, "a wave's SwiGLU columns are one 64-block");
     __shared__ __attribute__((aligned(1024))) uint16_t xs[3 * TT * G];
     __shared__ __attribute__((aligned(1024))) uint16_t wsm[NR * G];
     int& last_s = *reinterpret_cast<int*>(xs);             // after the k loop, whose last barrier frees xs
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l32 = lane & 31, h = lane >> 5, wt = wave >> 1, wn = wave & 1;
+    const int l16 = lane & 15, quarter = lane >> 4, wt = wave >> 1, wn = wave & 1;
     const int ntt = (T + TT - 1) / TT, ntn = (N + NC - 1) / NC, ntiles = ntt * ntn;
-    // Blocks are dealt round-robin to the 8 XCDs: each XCD takes a contiguous run of tiles, token
-    // tiles fastest, so that the blocks on one XCD share weight rows and pieces in its L2.
+    // Blocks are dealt round-robin to the 8 XCDs: each XCD takes a contiguous run of tiles, eight
+    // token tiles by all columns at a time, so that the blocks on one XCD share about as many
+    // pieces as weight rows in its L2.
     const int total = ntiles * S, xcd = blockIdx.x % 8;
     const int unit = xcd * (total / 8) + min(xcd, total % 8) + blockIdx.x / 8;
     const int tile = unit % ntiles, sp = unit / ntiles;
-    const int t0 = (tile % ntt) * TT, n0 = (tile / ntt) * NC;
+    const int band = tile / (8 * ntn), bt = min(8, ntt - 8 * band), in = tile - band * 8 * ntn;
+    const int t0 = (8 * band + in % bt) * TT, n0 = (in / bt) * NC;
     const int ng = K / G, g0 = sp * ng / S, g1 = (sp + 1) * ng / S;
 
     // Loads: each wave instruction brings eight rows of 128 bytes.  Rows past T or N repeat a
     // valid row and are never stored.
-    const int lr = lane >> 3, lc = 16 * ((lane & 7) ^ lr);
+    const int lr = lane >> 3, lc = 16 * ((lane & 7) ^ (4 * (wave & 1) + (lr >> 1)));
     int xo[2 * TF], wo[2 * NF];
 #pragma unroll
     for (int q = 0; q < 2 * TF; q++) xo[q] = min(t0 + 32 * q + 8 * wave + lr, T - 1) * (6 * K) + lc;
@@ -132,17 +136,25 @@ __device__ __forceinline__ void pf_mm(const uint16_t* __restrict__ W, const uint
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)X, (short)0, T * (6 * K), 0x00020000);
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
         (void*)W, (short)0, (EPI == EPI_SWIGLU ? 2 * N : N) * (2 * K), 0x00020000);
-    int tok[TF];                                           // this lane's tokens, clamped
+    int tok[TM];                                           // this lane's tokens, clamped
 #pragma unroll
-    for (int f = 0; f < TF; f++) tok[f] = min(t0 + 32 * (TF * wt + f) + l32, T - 1);
+    for (int f = 0; f < TM; f++) tok[f] = min(t0 + 32 * TF * wt + 16 * f + l16, T - 1);
 
-    f32x16 acc[TF][NF];
+    // acc[f][j]: tokens 16 * f.., weight rows 16 * j.. of the wave's part
+    sgpu_f32x4 acc[TM][NM];
 #pragma unroll
-    for (int f = 0; f < TF; f++)
+    for (int f = 0; f < TM; f++)
 #pragma unroll
-        for (int j = 0; j < NF; j++)
+        for (int j = 0; j < NM; j++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[f][j][r] = 0.0f;
+            for (int r = 0; r < 4; r++) acc[f][j][r] = 0.0f;
+    const int lrow = (lane & 15) * G, sw = (lane & 15) >> 1;      // operand reads: row lane % 16, swizzled chunk
+    const uint16_t* const xl = xs + 32 * TF * wt * G + lrow;
+    const uint16_t* const wl = wsm + 32 * NF * wn * G + lrow;
+    auto read_w = [&](int j, f16x8 (&w)[2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 2; s++) w[s] = *reinterpret_cast<const f16x8*>(wl + 16 * j * G + 8 * ((4 * s + quarter) ^ sw));
+    };
 
     for (int g = g0; g < g1; g++) {
         const int kb = g * (2 * G);
@@ -155,56 +167,69 @@ __device__ __forceinline__ void pf_mm(const uint16_t* __restrict__ W, const uint
 #pragma unroll
         for (int q = 0; q < 2 * NF; q++)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(wsm + (32 * q + 8 * wave) * G), 16, wo[q], kb, 0, 0);
-        float down[TF];
+        float down[TM];
 #pragma unroll
-        for (int f = 0; f < TF; f++) down[f] = xd[(size_t)tok[f] * ng + g];
+        for (int f = 0; f < TM; f++) down[f] = xd[(size_t)tok[f] * ng + g];
         __builtin_amdgcn_s_waitcnt(0);                     // this wave's rows are in LDS
         __syncthreads();
+        f16x8 w[2][2], x[2][3][2];
+        auto read_x = [&](int f) __attribute__((always_inline)) {
 #pragma unroll
-        for (int f = 0; f < TF; f++) {
-            f16x8 xf[3][4];
+            for (int p = 2; p >= 0; p--)
 #pragma unroll
-            for (int p = 0; p < 3; p++)
+                for (int s = 0; s < 2; s++)
 #pragma unroll
-                for (int s = 0; s < 4; s++)
-                    xf[p][s] = *reinterpret_cast<const f16x8*>(
-                        xs + (p * TT + 32 * (TF * wt + f) + l32) * G + 8 * ((2 * s + h) ^ (l32 & 7)));
+                    for (int u = 0; u < 2; u++)
+                        x[u][p][s] = *reinterpret_cast<const f16x8*>(xl + (p * TT + 16 * (f + u)) * G +
+                                                                     8 * ((4 * s + quarter) ^ sw));
+        };
+        read_w(0, w[0]);
+        read_x(0);
+        // one column of two 16x16 tiles per round: the next column's weights are read and the
+        // last one's sums are scaled under this one's products
+        sgpu_f32x4 c[2][2];
 #pragma unroll
-            for (int j = 0; j < NF; j++) {
-                f16x8 wf[4];
+        for (int i = 0; i <= TF * NM; i++) {
+            const int f = 2 * (i / NM), j = i % NM;
+            if (i < TF * NM) {
+                if (i + 1 < TF * NM) read_w((j + 1) % NM, w[(i + 1) % 2]);
 #pragma unroll
-                for (int s = 0; s < 4; s++)
-                    wf[s] = *reinterpret_cast<const f16x8*>(wsm + (32 * (NF * wn + j) + l32) * G +
-                                                            8 * ((2 * s + h) ^ (l32 & 7)));
-                f32x16 c;
-#pragma unroll
-                for (int r = 0; r < 16; r++) c[r] = 0.0f;
+                for (int u = 0; u < 2; u++) c[i % 2][u] = sgpu_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int p = 2; p >= 0; p--)
 #pragma unroll
-                    for (int s = 0; s < 4; s++) c = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[s], xf[p][s], c, 0, 0, 0);
+                    for (int s = 0; s < 2; s++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) acc[f][j][r] = __builtin_fmaf(c[r], down[f], acc[f][j][r]);
-                // no operand read ahead of its tile: the wave keeps within half a SIMD's registers,
-                // and the other block's wave has the matrix core meanwhile
-                __builtin_amdgcn_sched_barrier(0);
+                        for (int u = 0; u < 2; u++)
+                            c[i % 2][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[i % 2][s], x[u][p][s], c[i % 2][u], 0, 0, 0);
+                if (j == NM - 1 && i + 1 < TF * NM) read_x(f + 2);   // as the last products free their registers
             }
+            if (i > 0) {
+                const int f1 = 2 * ((i - 1) / NM), j1 = (i - 1) % NM;
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        acc[f1 + u][j1][r] = __builtin_fmaf(c[(i - 1) % 2][u][r], down[f1 + u], acc[f1 + u][j1][r]);
+            }
+            // rounds stay in order: the wave keeps within half a SIMD's registers
+            __builtin_amdgcn_sched_barrier(0);
         }
         __syncthreads();                                   // reads done before the next step's rows land
     }
 
-    // Accumulator r of tile (f, j): token tok[f], weight row 32 * (NF * wn + j) + 8 * (r / 4) +
-    // 4 * h + r % 4 of the block.
+    // Accumulator r of tile (f, j): token tok[f], weight row 32 * NF * wn + 16 * j + 4 * quarter + r
+    // of the block.
     if (EPI == EPI_STORE && S > 1) {
         constexpr int REC = 4096 * TF * NF;
         float* rec = ws + (size_t)(sp * ntiles + tile) * REC + tid;
 #pragma unroll
-        for (int f = 0; f < TF; f++)
+        for (int f = 0; f < TM; f++)
 #pragma unroll
-            for (int j = 0; j < NF; j++)
+            for (int j = 0; j < NM; j++)
 #pragma unroll
-                for (int r = 0; r < 16; r++)
-                    __hip_atomic_store(rec + ((f * NF + j) * 16 + r) * 256, acc[f][j][r], __ATOMIC_RELAXED,
+                for (int r = 0; r < 4; r++)
+                    __hip_atomic_store(rec + ((f * NM + j) * 4 + r) * 256, acc[f][j][r], __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT);
         __builtin_amdgcn_s_waitcnt(0);                     // this wave's partial stores are acknowledged
         __syncthreads();
@@ -214,91 +239,114 @@ __device__ __forceinline__ void pf_mm(const uint16_t* __restrict__ W, const uint
         }
         __syncthreads();
         if (!last_s) return;
-        // all splits in order, this block's own among them: a tile's loads of one split are issued
-        // before the first add
+        // all splits in order, this block's own among them, 16 loads issued before the first add
         for (int s2 = 0; s2 < S; s2++) {
             const float* src = ws + (size_t)(s2 * ntiles + tile) * REC + tid;
 #pragma unroll
-            for (int f = 0; f < TF; f++)
+            for (int f = 0; f < TM; f++)
 #pragma unroll
-                for (int j = 0; j < NF; j++) {
-                    f32x16 v;
+                for (int j = 0; j < NM; j += (NM < 4 ? NM : 4)) {
+                    sgpu_f32x4 v[NM < 4 ? NM : 4];
 #pragma unroll
-                    for (int r = 0; r < 16; r++)
-                        v[r] = __hip_atomic_load(src + ((f * NF + j) * 16 + r) * 256, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT);
+                    for (int i = 0; i < (NM < 4 ? NM : 4); i++)
 #pragma unroll
-                    for (int r = 0; r < 16; r++) acc[f][j][r] = s2 == 0 ? v[r] : acc[f][j][r] + v[r];
+                        for (int r = 0; r < 4; r++)
+                            v[i][r] = __hip_atomic_load(src + ((f * NM + j + i) * 4 + r) * 256, __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                    for (int i = 0; i < (NM < 4 ? NM : 4); i++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++) acc[f][j + i][r] = s2 == 0 ? v[i][r] : acc[f][j + i][r] + v[i][r];
                 }
         }
         if (tid == 0) __hip_atomic_store(cnt + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    const int tl = t0 + 32 * TF * wt + l32, nl = 32 * NF * wn + 4 * h;
-    if constexpr (EPI == EPI_STORE) {
+    const int tl = t0 + 32 * TF * wt + l16;
+    uint32_t top = 0;                                      // some sum non-finite: looked at once for the wave
 #pragma unroll
-        for (int f = 0; f < TF; f++) {
-            const int t = tl + 32 * f;
+    for (int f = 0; f < TM; f++)
+#pragma unroll
+        for (int j = 0; j < NM; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) top = max(top, __float_as_uint(acc[f][j][r]) & 0x7fffffffu);
+    const bool redo = __any(top >= 0x7f800000u);
+    if constexpr (EPI == EPI_STORE) {
+        const int nl = n0 + 32 * NF * wn + 4 * quarter;
+#pragma unroll
+        for (int f = 0; f < TM; f++) {
+            const int t = tl + 16 * f;
             if (t >= T) continue;
 #pragma unroll
-            for (int j = 0; j < NF; j++)
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const int n = n0 + nl + 32 * j + 8 * q;
-                    if (n >= N) continue;
-                    sgpu_f32x4 v;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        v[e] = acc[f][j][4 * q + e];
+            for (int j = 0; j < NM; j++) {
+                const int n = nl + 16 * j;
+                if (n >= N) continue;
+                sgpu_f32x4 v = acc[f][j];
+                if (redo) {
+                    for (int e = 0; e < 4; e++)
                         if (!__builtin_isfinite(v[e]))
                             v[e] = recompute(W + (size_t)(n + e) * K, X + (size_t)t * 3 * K, xd + (size_t)t * ng, K);
-                    }
-                    sgpu_f32x4* y = reinterpret_cast<sgpu_f32x4*>(Y + (size_t)t * N + n);
-                    if (bias) v += *reinterpret_cast<const sgpu_f32x4*>(bias + n);
-                    if (accum) v = *y + v;
-                    *y = v;
                 }
+                sgpu_f32x4* y = reinterpret_cast<sgpu_f32x4*>(Y + (size_t)t * N + n);
+                if (bias) v += *reinterpret_cast<const sgpu_f32x4*>(bias + n);
+                if (accum) v = *y + v;
+                *y = v;
+            }
         }
     } else {
 #pragma clang fp contract(off)
         const int c0 = n0 + 64 * wn;                       // the wave's 64 columns (whole: N % 64 == 0)
 #pragma unroll
-        for (int f = 0; f < TF; f++) {
-            const int t = tl + 32 * f;
+        for (int f = 0; f < TM; f++) {
+            const int t = tl + 16 * f;
             uint32_t m = 0;
+            if (redo) {
 #pragma unroll
-            for (int j = 0; j < 2; j++)
+                for (int j = 0; j < NM; j++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    float gt = acc[f][j][r], up = acc[f][j + 2][r];
-                    if (!__builtin_isfinite(gt) || !__builtin_isfinite(up)) {
-                        const int n = min(c0 + 32 * j + 8 * (r / 4) + 4 * h + r % 4, N - 1);
-                        const uint16_t* row = X + (size_t)min(t, T - 1) * 3 * K;
-                        const float* rd = xd + (size_t)min(t, T - 1) * ng;
-                        if (!__builtin_isfinite(gt)) gt = recompute(W + (size_t)n * K, row, rd, K);
-                        if (!__builtin_isfinite(up)) up = recompute(W + (size_t)(N + n) * K, row, rd, K);
-                    }
-                    const float v = (gt / (1.0f + expf(-gt))) * up;
+                    for (int r = 0; r < 4; r++)
+                        if (!__builtin_isfinite(acc[f][j][r])) {
+                            const int n = min(c0 + 16 * (j % 4) + 4 * quarter + r, N - 1);
+                            acc[f][j][r] = recompute(W + (size_t)(j < 4 ? n : N + n) * K, X + (size_t)min(t, T - 1) * 3 * K,
+                                                     xd + (size_t)min(t, T - 1) * ng, K);
+                        }
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float gt = acc[f][j][r], v = (gt / (1.0f + expf(-gt))) * acc[f][j + 4][r];
                     acc[f][j][r] = v;
                     m = max(m, mag_bits(v));
                 }
+            m = max(m, (uint32_t)__shfl_xor((int)m, 16));
             m = max(m, (uint32_t)__shfl_xor((int)m, 32));
-            if (t >= T || c0 >= N) continue;
             float up, down;
             block_scale(m, up, down);
-            if (h == 0) pd[(size_t)t * (N / G) + c0 / G] = down;
-            uint16_t* row = P + (size_t)t * 3 * N + c0 + 4 * h;
+            // through LDS (the wave's own 6 KB, free after the k loop) so that a row's 64 codes of
+            // a piece leave as one 128-byte line: 8-byte stores straight from the accumulators
+            // made it 175 us instead of 171 at 3001 rows
+            uint16_t* const st = xs + wave * (3 * 16 * G);
 #pragma unroll
-            for (int j = 0; j < 2; j++)
+            for (int j = 0; j < 4; j++) {
+                const float x[4] = {acc[f][j][0], acc[f][j][1], acc[f][j][2], acc[f][j][3]};
+                f16x4 p[3];
+                split3(x, up, p[0], p[1], p[2]);
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const float x[4] = {acc[f][j][4 * q], acc[f][j][4 * q + 1], acc[f][j][4 * q + 2], acc[f][j][4 * q + 3]};
-                    f16x4 p0, p1, p2;
-                    split3(x, up, p0, p1, p2);
-                    uint16_t* d = row + 32 * j + 8 * q;
-                    *reinterpret_cast<f16x4*>(d) = p0;
-                    *reinterpret_cast<f16x4*>(d + N) = p1;
-                    *reinterpret_cast<f16x4*>(d + 2 * N) = p2;
+                for (int q = 0; q < 3; q++)
+                    *reinterpret_cast<f16x4*>(st + (16 * q + l16) * G + 8 * ((2 * j + quarter / 2) ^ sw) + 4 * (quarter & 1)) = p[q];
+            }
+            sgpu::wave_sync();
+            if (t < T && c0 < N && quarter == 0) pd[(size_t)t * (N / G) + c0 / G] = down;
+#pragma unroll
+            for (int q = 0; q < 3; q++)
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    const int r = 8 * i + lr, tr = t0 + 32 * TF * wt + 16 * f + r, ch = lane & 7;
+                    const sgpu_u32x4 v = *reinterpret_cast<const sgpu_u32x4*>(st + (16 * q + r) * G + 8 * (ch ^ (r >> 1)));
+                    if (tr < T && c0 < N)
+                        *reinterpret_cast<sgpu_u32x4*>(P + (size_t)tr * 3 * N + (size_t)q * N + c0 + 8 * ch) = v;
                 }
+            sgpu::wave_sync();
         }
     }
 }
@@ -579,15 +627,14 @@ SGPU_PF_ATTN(128)
         unsigned* __restrict__ cnt, int accum) {                                                                      \
         pf_mm<TF, NF, EPI_STORE>(W, X, xd, bias, Y, nullptr, nullptr, K, N, T, S, ws, cnt, accum);                    \
     }
-#define SGPU_PF_GATEUP(TF)                                                                                            \
-    extern "C" __global__ void __launch_bounds__(256, 2) sgpu_pf_gateup_##TF(                                         \
-        const uint16_t* __restrict__ W, const uint16_t* __restrict__ X, const float* __restrict__ xd,                 \
-        uint16_t* __restrict__ P, float* __restrict__ pd, int K, int N, int T) {                                      \
-        pf_mm<TF, 4, EPI_SWIGLU>(W, X, xd, nullptr, nullptr, P, pd, K, N, T, 1, nullptr, nullptr, 0);                 \
-    }
+// 64 tokens and 128 SwiGLU columns a block.  128 tokens a block were slower at every prompt length
+// (Qwen2.5-0.5B: 36 us against 53 at 500 rows, 151 against 156 at 3001): a CU holds two blocks
+// of either, and the smaller one's step waits for 56 KB instead of 80.
+extern "C" __global__ void __launch_bounds__(256, 2) sgpu_pf_gateup(
+    const uint16_t* __restrict__ W, const uint16_t* __restrict__ X, const float* __restrict__ xd,
+    uint16_t* __restrict__ P, float* __restrict__ pd, int K, int N, int T) {
+    pf_mm<1, 4, EPI_SWIGLU>(W, X, xd, nullptr, nullptr, P, pd, K, N, T, 1, nullptr, nullptr, 0);
+}
 SGPU_PF_MM(1, 1)
 SGPU_PF_MM(1, 2)
 SGPU_PF_MM(2, 2)
-SGPU_PF_MM(2, 4)
-SGPU_PF_GATEUP(1)
-SGPU_PF_GATEUP(2)

@@ -29,7 +29,7 @@ KERNELS = [
     ("switch_gpu", "sgemm_splitk"),              # split-K SGEMM (also the allocation-free entry)
     ("gpt2_kernels", "gemv_multi_splitk"),       # the split batched GEMM
     ("sgpu_decode", "sgpu_pf_gemm"),             # the Qwen prefill's split GEMM
-    ("sgpu_prefill", "sgpu_pf_mm_24"),           # the prompt products in fp16 pieces, split
+    ("sgpu_prefill", "sgpu_pf_mm_22"),           # the prompt products in fp16 pieces, split
     ("sgpu_prefill", "sgpu_pf_mm_11"),
     ("sgpu_decode", "sgpu_dec_attn32"),          # decode attention, chunked caches
     ("sgpu_decode", "sgpu_dec_attn64"),
