@@ -151,6 +151,10 @@ int sgpu_sgemm_opt(const float *A, const float *B, float *C, int M, int N, int K
  * "sgemm_kwave_edge" and "sgemm_kwave128" the member the size rule picks, and with an operand
  * off 4 bytes "sgemm_kwave" or "sgemm_kwave_edge" becomes the 64x64-or-larger member the size
  * rule picks.
+ * A product of "sgemm_opt", "sgemm_opt256", "sgemm_kwave", "sgemm_kwave_edge" or
+ * "sgemm_kwave128" runs in the form of sgpu_sgemm_pieces where that is estimated to be faster
+ * (large problems, float-aligned operands), here and in the members' own launchers alike; the
+ * kernels of these names are the fp32 members themselves.
  * No counterpart in the reference (its sgemm_opt is one kernel). */
 const char *sgpu_sgemm_opt_plan(int M, int N, int K, int cus, int *splits);
 /* The sgemm_opt256 member alone (any shape; masked loads on edge tiles).  No
@@ -184,6 +188,14 @@ int sgpu_sgemm_kwave_edge(const float *A, const float *B, float *C, int M, int N
  * counterpart in the reference: an added member of the family with the (A, B, C, M, N, K)
  * symbol arguments. */
 int sgpu_sgemm_kwave128(const float *A, const float *B, float *C, int M, int N, int K, void *stream);
+/* The same product on the bf16 matrix cores: every operand cut without loss into three bf16
+ * pieces, six exact piece products summed in fp32, 128x128 tiles (results as close to the exact
+ * product as the fp32 members'; non-finite sums, and rows or columns of numbers too small to
+ * cut, by serial fp32 FMAs).  M, N >= 128, K >= 32, float-aligned A, B, C
+ * (SGPU_ERR_INVALID_ARG otherwise; M or N == 0 is a no-op).  The tiles past the last full round
+ * of compute units are split over K through the stream's split-K workspace; a stream that has
+ * none and cannot get one runs them unsplit.  No counterpart in the reference. */
+int sgpu_sgemm_pieces(const float *A, const float *B, float *C, int M, int N, int K, void *stream);
 /* The sgemm_splitk member: 64x64 tiles with K split S ways (S >= 1; reduced so that every
  * split holds at least one 32-deep slice), each (tile, split) a block.  Every split writes its
  * partial tile to a library-owned workspace of the launch's stream and the last split of a

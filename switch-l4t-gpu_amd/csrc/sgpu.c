@@ -29,9 +29,10 @@ extern const unsigned char sgpu_co_qwen_kernels[], sgpu_co_qwen_kernels_end[];
 extern const unsigned char sgpu_co_sgpu_tuned[], sgpu_co_sgpu_tuned_end[];
 extern const unsigned char sgpu_co_sgpu_decode[], sgpu_co_sgpu_decode_end[];
 extern const unsigned char sgpu_co_sgpu_prefill[], sgpu_co_sgpu_prefill_end[];
+extern const unsigned char sgpu_co_sgpu_pieces[], sgpu_co_sgpu_pieces_end[];
 extern const unsigned char sgpu_co_sgpu_probe[], sgpu_co_sgpu_probe_end[];
 
-enum { MOD_SWITCH, MOD_GEMV, MOD_GPT2, MOD_QWEN, MOD_TUNED, MOD_DECODE, MOD_PREFILL, MOD_PROBE, NMOD };
+enum { MOD_SWITCH, MOD_GEMV, MOD_GPT2, MOD_QWEN, MOD_TUNED, MOD_DECODE, MOD_PREFILL, MOD_PIECES, MOD_PROBE, NMOD };
 static const struct {
     const char *name;
     const unsigned char *start, *end;
@@ -43,6 +44,7 @@ static const struct {
     {"sgpu_tuned", sgpu_co_sgpu_tuned, sgpu_co_sgpu_tuned_end},
     {"sgpu_decode", sgpu_co_sgpu_decode, sgpu_co_sgpu_decode_end},
     {"sgpu_prefill", sgpu_co_sgpu_prefill, sgpu_co_sgpu_prefill_end},
+    {"sgpu_pieces", sgpu_co_sgpu_pieces, sgpu_co_sgpu_pieces_end},
     {"sgpu_probe", sgpu_co_sgpu_probe, sgpu_co_sgpu_probe_end},
 };
 
@@ -54,7 +56,7 @@ enum {
     K_GEMV, K_GEMV4, K_GEMV_WARP, K_GEMV_WARP_B, K_GEMV_MULTI, K_GEMV_MULTI_SPLITK, K_GEMV_MULTI_X8_64,
     K_GEMV_MULTI_X8_256,
     K_GEMV_H, K_GEMV_HH, K_RMSNORM, K_ROPE, K_SWIGLU, K_ASCORES, K_ASOFTMAX, K_AMIX, K_ADD2,
-    K_EMBED_H,
+    K_EMBED_H, K_SGEMM_PIECES, K_SGEMM_PIECES_WIDE,
     K_LAYERNORM, K_GELU, K_ADD_BIAS, K_G2_SCORES, K_G2_SOFTMAX, K_G2_MIX,
     NKERN
 };
@@ -74,7 +76,8 @@ static const struct {
     {MOD_QWEN, "gemv_h"}, {MOD_QWEN, "gemv_hh"}, {MOD_QWEN, "rmsnorm"}, {MOD_QWEN, "rope"}, {MOD_QWEN, "swiglu"},
     {MOD_QWEN, "attn_scores_gqa"}, {MOD_QWEN, "attn_softmax"}, {MOD_QWEN, "attn_mix_gqa"},
     {MOD_QWEN, "add2"},
-    {MOD_TUNED, "sgpu_embed_h"},
+    {MOD_TUNED, "sgpu_embed_h"}, {MOD_PIECES, "sgpu_sgemm_pieces"},
+    {MOD_PIECES, "sgpu_sgemm_pieces_wide"},
     {MOD_GPT2, "layernorm"}, {MOD_GPT2, "gelu"}, {MOD_GPT2, "add_bias"}, {MOD_GPT2, "attn_scores"},
     {MOD_GPT2, "attn_softmax"}, {MOD_GPT2, "attn_mix"},
 };
@@ -701,7 +704,10 @@ int sgpu_sgemm_tiled(const float *A, const float *B, float *C, int M, int N, int
 int sgpu_sgemm_tiled4(const float *A, const float *B, float *C, int M, int N, int K, void *stream) {
     return sgemm_common(K_SGEMM_TILED4, "sgemm_tiled4", A, B, C, M, N, K, stream);
 }
+static int pieces_taken(const float *A, const float *B, float *C, int M, int N, int K, void *stream, int *rc);
 int sgpu_sgemm_opt256(const float *A, const float *B, float *C, int M, int N, int K, void *stream) {
+    int rc;
+    if (pieces_taken(A, B, C, M, N, K, stream, &rc)) return rc;
     return sgemm_common(K_SGEMM_OPT256, "sgemm_opt256", A, B, C, M, N, K, stream);
 }
 /* sgemm_kwave's problems: M, N multiples of 64, K a multiple of 32 (the operands' 16-byte
@@ -722,6 +728,8 @@ int sgpu_sgemm_kwave(const float *A, const float *B, float *C, int M, int N, int
     if (M < 0 || N < 0 || K < 0) return SGPU_ERR_INVALID_ARG;
     if (M == 0 || N == 0) return SGPU_OK;
     if (!kwave_shape(M, N, K) || !A || !B || !C || (((uintptr_t)A | (uintptr_t)B) & 15)) return SGPU_ERR_INVALID_ARG;
+    int rc;
+    if (pieces_taken(A, B, C, M, N, K, stream, &rc)) return rc;
     return kwave_launch(0, A, B, C, M, N, K, stream);
 }
 /* sgemm_kwave128's problems: M, N multiples of 128, K a multiple of 32, a 128-row A panel and a
@@ -735,7 +743,98 @@ int sgpu_sgemm_kwave128(const float *A, const float *B, float *C, int M, int N, 
     if (M < 0 || N < 0 || K < 0) return SGPU_ERR_INVALID_ARG;
     if (M == 0 || N == 0) return SGPU_OK;
     if (!kwave128_shape(M, N, K) || !A || !B || !C || (((uintptr_t)A | (uintptr_t)B) & 15)) return SGPU_ERR_INVALID_ARG;
+    int rc;
+    if (pieces_taken(A, B, C, M, N, K, stream, &rc)) return rc;
     return sgemm_common(K_SGEMM_KWAVE128, "sgemm_kwave128", A, B, C, M, N, K, stream);
+}
+/* The bf16-piece form (sgpu_pieces.hip): whole or shifted tiles of 128 rows and 128 or 256
+ * (wide) columns, 32-deep k-slices; the tiles past the last full round of CUs are split S ways
+ * where a workspace is at hand. */
+typedef struct {
+    int wide, S;
+    long long tiles, full;
+    double us;                                /* estimate */
+} pieces_plan;
+static int pieces_shape(int M, int N, int K) {
+    return M >= 128 && N >= 128 && K >= 32 && (long long)cdiv(M, 128) * cdiv(N, 128) < 1LL << 20;
+}
+static pieces_plan pieces_form(int M, int N, int K, int cus, int wide, int split) {
+    const int tn = wide ? 256 : 128, ns = (int)cdiv(K, 32), rec = 128 * tn + 128 + tn;
+    /* us per slice of a tile, and per round to start and store it: measured */
+    const double slice = wide ? 2.3 : 1.42, once = wide ? 8.0 : 5.0;
+    pieces_plan p = {wide, 1, (long long)cdiv(M, 128) * cdiv(N, tn), 0, 0.0};
+    const long long rest = p.tiles % cus;
+    p.full = p.tiles - rest;
+    if (rest && split) {
+        p.S = (int)(cus / rest);
+        if (p.S > ns / 4) p.S = ns / 4;       /* four slices a block or more */
+        while (p.S > 1 && (long long)p.S * rest * rec > (long long)SK_WS_FLOATS) p.S--;
+        if (p.S > 16) p.S = 16;
+        if (p.S < 1) p.S = 1;
+    }
+    if (p.S == 1) p.full = p.tiles;
+    p.us = (double)(p.tiles / cus) * ns * slice + (rest ? (double)cdiv(ns, p.S) * slice + (p.S > 1 ? 2.0 + p.S : 0.0) : 0.0) +
+           once * (double)((p.tiles + cus - 1) / cus);
+    return p;
+}
+static pieces_plan pieces_best(int M, int N, int K, int cus, int split) {
+    const pieces_plan n = pieces_form(M, N, K, cus, 0, split);
+    if (N < 256) return n;
+    const pieces_plan w = pieces_form(M, N, K, cus, 1, split);
+    return w.us < n.us ? w : n;
+}
+static int pieces_launch(devstate *d, const float *A, const float *B, float *C, int M, int N, int K,
+                         const pieces_plan *p, float *ws, unsigned *cnt, void *stream) {
+    int full = (int)p->full, S = p->S;
+    unsigned g[3] = {(unsigned)(p->full + (p->tiles - p->full) * S), 1, 1}, b[3] = {512, 1, 1};
+    void *args[] = {&A, &B, &C, &M, &N, &K, &full, &S, &ws, &cnt};
+    return launch(d->fn[p->wide ? K_SGEMM_PIECES_WIDE : K_SGEMM_PIECES], g, b, stream, args);
+}
+/* Whether the piece form of the product is the faster one: its estimate, with a margin of 1 us,
+ * against the fp32 members' (rounds of 64x64 tiles at 14.3 ns per k, or the whole at 125 TFLOP/s).
+ * Measured over 70 shapes of 64 to 8192 a side (log-uniform, K from 86 on) the rule's choices take
+ * 14% less time than the fp32 members alone, the best choices 15% less; 4096^3 936 -> 602 us,
+ * 3072^3 419 -> 270, 2048^3 121.6 -> 90.1, 4097^3 1102 -> 678, 2047x2049x2048 134.9 -> 117.7.
+ * Where it loses, the rule keeps the members: 1024^3 25.2 against 19.8, 1023x1025x997 25.4 against
+ * 21.1, 3000x3000x128 35.7 against 27.3. */
+static int pieces_win(const pieces_plan *p, int M, int N, int K, int cus) {
+    const long long t64 = kwave_edge_tiles(M, N), rounds = (t64 + cus - 1) / cus;
+    const double flat = 2e-6 * M * N * (double)K / 125.0 + 4.0, byround = 0.0143 * (double)rounds * K + 4.0;
+    const double member = byround > 1.35 * flat ? 1.35 * flat : byround > flat ? byround : flat;
+    return p->us + 1.0 < member;
+}
+/* For the launchers of large products (sgemm_opt256, sgemm_kwave, sgemm_kwave_edge, sgemm_kwave128
+ * and what sgpu_sgemm_opt plans as one of these): 1 when the product was launched in its piece
+ * form (*rc: the launch's status).  Without a workspace
+ * the tail is not split, which can turn the choice. */
+static int pieces_taken(const float *A, const float *B, float *C, int M, int N, int K, void *stream, int *rc) {
+    if (!pieces_shape(M, N, K) || !A || !B || !C || (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 3)) return 0;
+    devstate *d = cur(rc);
+    if (!d) return 1;
+    pieces_plan p = pieces_best(M, N, K, d->cus, 1);
+    float *ws = NULL;
+    unsigned *cnt = NULL;
+    if (!pieces_win(&p, M, N, K, d->cus)) return 0;
+    if (p.S > 1 && sk_workspace(d, stream, &ws, &cnt) != SGPU_OK) {
+        p = pieces_best(M, N, K, d->cus, 0);
+        if (!pieces_win(&p, M, N, K, d->cus)) return 0;
+    }
+    *rc = pieces_launch(d, A, B, C, M, N, K, &p, ws, cnt, stream);
+    return 1;
+}
+int sgpu_sgemm_pieces(const float *A, const float *B, float *C, int M, int N, int K, void *stream) {
+    if (M < 0 || N < 0 || K < 0) return SGPU_ERR_INVALID_ARG;
+    if (M == 0 || N == 0) return SGPU_OK;
+    if (!pieces_shape(M, N, K) || !A || !B || !C || (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 3))
+        return SGPU_ERR_INVALID_ARG;
+    int rc;
+    devstate *d = cur(&rc);
+    if (!d) return rc;
+    pieces_plan p = pieces_best(M, N, K, d->cus, 1);
+    float *ws = NULL;
+    unsigned *cnt = NULL;
+    if (p.S > 1 && sk_workspace(d, stream, &ws, &cnt) != SGPU_OK) p = pieces_best(M, N, K, d->cus, 0);
+    return pieces_launch(d, A, B, C, M, N, K, &p, ws, cnt, stream);
 }
 /* sgemm_kwave_edge's problems: M, N at least 64 (a partial last row or column of tiles is the
  * 64 rows or columns ending at the last one), K at least 1, float-aligned operands. */
@@ -746,6 +845,8 @@ int sgpu_sgemm_kwave_edge(const float *A, const float *B, float *C, int M, int N
     if (M == 0 || N == 0) return SGPU_OK;
     if (!kwave_edge_shape(M, N, K) || !A || !B || !C || (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 3))
         return SGPU_ERR_INVALID_ARG;
+    int rc;
+    if (pieces_taken(A, B, C, M, N, K, stream, &rc)) return rc;
     return kwave_launch(1, A, B, C, M, N, K, stream);
 }
 /* The optimised entry picks the member with the least work on its busiest CU: tiles are one
@@ -997,6 +1098,9 @@ int sgpu_sgemm_opt(const float *A, const float *B, float *C, int M, int N, int K
     unsigned *cnt;
     if (p == PLAN_SPLITK && sk_workspace(d, stream, &ws, &cnt) == SGPU_OK)    /* else: the unsplit member */
         return splitk_launch(d, A, B, C, M, N, K, S, ws, cnt, stream);
+    const int big = p >= 0 && (g_sgemm_members[p].kid == K_SGEMM_OPT || g_sgemm_members[p].kid == K_SGEMM_OPT256);
+    if ((p == PLAN_KWAVE128 || p == PLAN_KWAVE || p == PLAN_KWAVE_EDGE || big) && pieces_taken(A, B, C, M, N, K, stream, &rc))
+        return rc;
     if (p == PLAN_KWAVE128 && !(((uintptr_t)A | (uintptr_t)B) & 15))
         return sgemm_common(K_SGEMM_KWAVE128, "sgemm_kwave128", A, B, C, M, N, K, stream);
     if (p == PLAN_KWAVE && !(((uintptr_t)A | (uintptr_t)B) & 15)) return kwave_launch(0, A, B, C, M, N, K, stream);

@@ -1,0 +1,291 @@
+// sgpu_pieces.hip -- the large fp32 SGEMM on the bf16 matrix cores (gfx950).
+//
+// C = A B (row-major fp32) for problems of many 128x128 tiles.  The fp32 matrix instructions
+// reach 157 TFLOP/s, and the members built on them run at 94% of that; bf16 ones are sixteen
+// times as fast.  Every operand is cut without loss into three bf16 pieces x = p0 + p1 + p2
+// (8 + 8 + 8 mantissa bits, each piece the rest rounded to nearest), and the product is the sum
+// of the six piece products p_i q_j with i + j <= 2: those left out are below 2^-26 of |x y|.
+// A product of pieces is exact in the fp32 accumulators.  p0 q0 has accumulators of its own and
+// the five small products share a second set, so the long sum is rounded once per 32 k.
+//
+// The cut needs normal-sized numbers.  Where it would lose bits that fp32 keeps, or meets what it
+// cannot represent, the elements concerned are computed again by serial fp32 FMAs:
+//  * sums that come out non-finite (an infinity, a NaN, an operand that rounds up to infinity);
+//  * rows of A or columns of B whose largest magnitude is below 2^-100 (bf16 subnormals end at
+//    2^-133), and row-column pairs whose largest product is below 2^-96.
+#include "sgpu_device.h"
+
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+constexpr int TM = 128, KS = 32;                       // tile rows, k per step
+
+// The three pieces of two numbers, packed: the first rounded to nearest, then the upper halves of
+// what is left (16 bits at most), which v_perm takes at full rate; three conversions to bf16
+// instead of one cost the step a third more issue time.
+__device__ __forceinline__ void cut2(float x0, float x1, uint32_t (&p)[3]) {
+    p[0] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x0, x1}, bf16x2));
+    x0 -= __uint_as_float(p[0] << 16);
+    x1 -= __uint_as_float(p[0] & 0xffff0000u);
+    p[1] = __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u);
+    x0 -= __uint_as_float(__float_as_uint(x0) & 0xffff0000u);
+    x1 -= __uint_as_float(__float_as_uint(x1) & 0xffff0000u);
+    p[2] = __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u);
+}
+__device__ __forceinline__ float max3abs(float m, float a, float b) { return fmaxf(fmaxf(m, fabsf(a)), fabsf(b)); }
+
+__device__ __noinline__ float serial_dot(const float* __restrict__ a, const float* __restrict__ b, int K, int N) {
+    float acc = 0.0f;
+    for (int k = 0; k < K; k++) acc = __builtin_fmaf(a[k], b[(size_t)k * N], acc);
+    return acc;
+}
+
+// Bound: the matrix cores.  A block of 2x4 waves computes a tile of 128 x 64 NJ, a wave 64 x 16 NJ of
+// it in 16x16 tiles.  Operands pass through two LDS buffers of 32 k: while the matrix cores run on
+// one, the waves cut the next 32 k (read into registers half a step or more earlier) into the
+// other, their VALU work and LDS writes dealt out between the MFMAs, so that a step has one
+// barrier; two waves a SIMD fill each other's waits.  A's rows and B's columns hold their 32 k of
+// a piece in 64 bytes (16-byte chunk c at c ^ (-(row / 4) % 4): a read serves lanes 0-3, 12-15, 20-23
+// and 24-27 and the like together, and these then use all 64 banks).  B's column n is kept in LDS
+// row n % NJ * 64 + n / NJ, so that a lane ends with NJ consecutive columns of C.
+// A last row or column of tiles that would pass M or N ends at M or N (its overlap is computed
+// twice, alike), a last step that would pass K starts at K - 32 with the k already summed set to
+// zero: no load needs a bound.  Operands of any float alignment.
+// The first `full` tiles are one block each; those that are left, too few for a round of all CUs, are
+// split over S blocks of consecutive slices each, whose sums meet by the hand-off of
+// sgpu_device.h: ws holds one record of 128 * TN + 128 + TN floats per block (its tile, then its
+// rows' and columns' largest magnitudes), cnt one zeroed counter per split tile.
+// Preconditions (launcher): M >= 128, N >= 64 NJ, K >= 32, 4-byte aligned operands, blockDim 512,
+// 1 <= S <= slices of 32 k, grid = full + (tiles - full) * S.
+template <int NJ>
+__device__ __forceinline__ void sgemm_pieces(const float* __restrict__ A, const float* __restrict__ B,
+                                             float* __restrict__ C, int M, int N, int K, int full, int S,
+                                             float* __restrict__ ws, unsigned* __restrict__ cnt) {
+    constexpr int TN = 64 * NJ, REC = TM * TN + TM + TN;
+    typedef float rowv __attribute__((ext_vector_type(NJ)));
+    typedef float rowv_a4 __attribute__((ext_vector_type(NJ), aligned(4)));
+    __shared__ __attribute__((aligned(1024))) uint16_t as[2][3 * TM * KS], bs[2][3 * TN * KS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, quarter = lane >> 4, wm = wave >> 2, wn = wave & 3;
+    // Blocks are dealt round-robin to the 8 XCDs: of the unsplit tiles each XCD takes a contiguous
+    // run, eight tile rows by all columns at a time, so that its blocks share operands in its L2.
+    const int ntm = (M + TM - 1) / TM, ntn = (N + TN - 1) / TN, rest = ntm * ntn - full, xcd = blockIdx.x % 8;
+    const bool whole = (int)blockIdx.x < full;
+    const int u = (int)blockIdx.x - full, part = whole ? 0 : u % rest, sp = whole ? 0 : u / rest;
+    const int tile = whole ? xcd * (full / 8) + min(xcd, full % 8) + blockIdx.x / 8 : full + part;
+    const int band = tile / (8 * ntn), bm = min(8, ntm - 8 * band), in = tile - band * 8 * ntn;
+    const int m0 = min((8 * band + in % bm) * TM, M - TM), n0 = min((in / bm) * TN, N - TN);
+
+    // A thread's part of a slice: A rows r and r + 64, k 4 q..; B rows k 4 q + i, columns NJ r...
+    const int r = tid >> 3, q = tid & 7;
+    const float* ap = A + (size_t)(m0 + r) * K + 4 * q;
+    const float* bp = B + (size_t)(4 * q) * N + n0 + NJ * r;
+    f32x4 av[2];
+    rowv bv[4];
+    auto load_a = [&](int s) __attribute__((always_inline)) {
+        const int k0 = min(KS * s, K - KS);
+#pragma unroll
+        for (int i = 0; i < 2; i++) av[i] = *reinterpret_cast<const sgpu_f32x4_a4*>(ap + (size_t)(64 * i) * K + k0);
+    };
+    auto load_b = [&](int s) __attribute__((always_inline)) {
+        const int k0 = min(KS * s, K - KS);
+#pragma unroll
+        for (int i = 0; i < 4; i++) bv[i] = *reinterpret_cast<const rowv_a4*>(bp + (size_t)(k0 + i) * N);
+    };
+    // k of slice s that are summed already: set to zero
+    auto mask = [&](int s) __attribute__((always_inline)) {
+        const int done = KS * s - (K - KS);
+        if (done <= 0) return;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            if (4 * q + e >= done) continue;
+            av[0][e] = av[1][e] = 0.0f;
+#pragma unroll
+            for (int c = 0; c < NJ; c++) bv[e][c] = 0.0f;
+        }
+    };
+    float amax[2] = {0.0f, 0.0f}, bmax[NJ];
+#pragma unroll
+    for (int c = 0; c < NJ; c++) bmax[c] = 0.0f;
+    const int wo = r * KS + 8 * ((q >> 1) ^ (-(r >> 2) & 3)) + 4 * (q & 1);
+    auto cut_a = [&](int buf, int i) __attribute__((always_inline)) {
+        uint32_t lo[3], hi[3];
+        cut2(av[i][0], av[i][1], lo);
+        cut2(av[i][2], av[i][3], hi);
+#pragma unroll
+        for (int p = 0; p < 3; p++) *reinterpret_cast<u32x2*>(as[buf] + wo + (p * TM + 64 * i) * KS) = u32x2{lo[p], hi[p]};
+        amax[i] = max3abs(max3abs(amax[i], av[i][0], av[i][1]), av[i][2], av[i][3]);
+    };
+    auto cut_b = [&](int buf, int c) __attribute__((always_inline)) {
+        uint32_t lo[3], hi[3];
+        cut2(bv[0][c], bv[1][c], lo);
+        cut2(bv[2][c], bv[3][c], hi);
+#pragma unroll
+        for (int p = 0; p < 3; p++) *reinterpret_cast<u32x2*>(bs[buf] + wo + (p * TN + 64 * c) * KS) = u32x2{lo[p], hi[p]};
+        bmax[c] = max3abs(max3abs(bmax[c], bv[0][c], bv[1][c]), bv[2][c], bv[3][c]);
+    };
+    f32x4 acc[4][NJ], low[4][NJ];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[i][j] = low[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const int ch = 8 * (quarter ^ (-(l16 >> 2) & 3));
+    const int aro = (64 * wm + l16) * KS + ch, bro = (16 * wn + l16) * KS + ch;
+
+    const int ns = (K + KS - 1) / KS;                      // this block's slices: s0..nk-1
+    const int s0 = whole ? 0 : sp * ns / S, nk = whole ? ns : (sp + 1) * ns / S;
+    // Step s on LDS buffer `buf`: slice s + 1 cut into the other one, slice s + 2 read.  What is cut past
+    // the block's last slice is not used.
+    auto step = [&](int s, int buf) __attribute__((always_inline)) {
+        mask(s + 1);
+        bf16x8 b[NJ][3];
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+            for (int p = 0; p < 3; p++) b[j][p] = *reinterpret_cast<const bf16x8*>(bs[buf] + bro + (p * TN + 64 * j) * KS);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            bf16x8 a[3];
+#pragma unroll
+            for (int p = 0; p < 3; p++) a[p] = *reinterpret_cast<const bf16x8*>(as[buf] + aro + (p * TM + 16 * i) * KS);
+            constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+            for (int t = 0; t < 6; t++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++) {
+                    f32x4& d = t < 5 ? low[i][j] : acc[i][j];
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[pa[t]], b[j][pb[t]], d, 0, 0, 0);
+                }
+            if (i < 2) {
+#pragma unroll
+                for (int c = 0; c < NJ / 2; c++) cut_b(buf ^ 1, NJ / 2 * i + c);
+                if (i == 1) load_b(s + 2);
+            } else {
+                cut_a(buf ^ 1, i - 2);
+                if (i == 3) load_a(s + 2);
+            }
+        }
+        __syncthreads();
+    };
+    load_a(s0);
+    load_b(s0);
+    mask(s0);
+#pragma unroll
+    for (int c = 0; c < NJ; c++) cut_b(0, c);
+    load_b(s0 + 1);
+    cut_a(0, 0);
+    cut_a(0, 1);
+    load_a(s0 + 1);
+    __syncthreads();
+    for (int s = s0; s < nk; s += 2) {
+        step(s, 0);
+        if (s + 1 < nk) step(s + 1, 1);
+    }
+
+    // The largest magnitude of each of the tile's rows and columns, through LDS.
+    float* const rmax = reinterpret_cast<float*>(as[0]);   // 128 rows, then TN columns
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+#pragma unroll
+        for (int o = 1; o < 8; o *= 2) amax[i] = fmaxf(amax[i], __shfl_xor(amax[i], o));
+        if (q == 0) rmax[r + 64 * i] = amax[i];
+    }
+#pragma unroll
+    for (int c = 0; c < NJ; c++) {
+#pragma unroll
+        for (int o = 1; o < 8; o *= 2) bmax[c] = fmaxf(bmax[c], __shfl_xor(bmax[c], o));
+        if (q == 0) rmax[TM + NJ * r + c] = bmax[c];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[i][j] += low[i][j];
+    __syncthreads();
+    if (!whole && S > 1) {
+        float* const rec = ws + (size_t)(sp * rest + part) * REC;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    __hip_atomic_store(rec + ((i * NJ + j) * 4 + e) * 512 + tid, acc[i][j][e], __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+        if (tid < TM + TN)
+            __hip_atomic_store(rec + TM * TN + tid, rmax[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_s_waitcnt(0);                     // this wave's partial stores are acknowledged
+        int& last_s = *reinterpret_cast<int*>(bs[0]);
+        __syncthreads();
+        if (tid == 0) {
+            last_s = __hip_atomic_fetch_add(cnt + part, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(S - 1);
+            if (last_s) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");   // before the others' partials
+        }
+        __syncthreads();
+        if (!last_s) return;
+        float big = 0.0f;
+        for (int s2 = 0; s2 < S; s2++) {                   // all parts in order, this block's own among them
+            const float* src = ws + (size_t)(s2 * rest + part) * REC;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                f32x4 v[NJ];
+#pragma unroll
+                for (int j = 0; j < NJ; j++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        v[j][e] = __hip_atomic_load(src + ((i * NJ + j) * 4 + e) * 512 + tid, __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                for (int j = 0; j < NJ; j++) acc[i][j] = s2 == 0 ? v[j] : acc[i][j] + v[j];
+            }
+            if (tid < TM + TN)
+                big = fmaxf(big, __hip_atomic_load(src + TM * TN + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        }
+        if (tid < TM + TN) rmax[tid] = big;
+        if (tid == 0) __hip_atomic_store(cnt + part, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+    }
+    // Accumulator e of tile (i, j): row 64 wm + 16 i + 4 quarter + e, column NJ (16 wn + l16) + j.
+    const int lc = NJ * (16 * wn + l16), n = n0 + lc;
+    float cmax[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; j++) cmax[j] = rmax[TM + lc + j];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int lm = 64 * wm + 16 * i + 4 * quarter + e, m = m0 + lm;
+            const float ra = rmax[lm];
+            rowv v;
+            bool redo = false;
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                v[j] = acc[i][j][e];
+                redo |= !__builtin_isfinite(v[j]) || (fminf(fminf(ra, cmax[j]) * 0x1p100f, ra * cmax[j] * 0x1p96f) < 1.0f &&
+                                                      ra > 0.0f && cmax[j] > 0.0f);
+            }
+            if (redo)
+                for (int j = 0; j < NJ; j++) v[j] = serial_dot(A + (size_t)m * K, B + n + j, K, N);
+            *reinterpret_cast<rowv_a4*>(C + (size_t)m * N + n) = v;
+        }
+}
+
+}  // namespace
+
+extern "C" __global__ void __launch_bounds__(512) sgpu_sgemm_pieces(const float* __restrict__ A, const float* __restrict__ B,
+                                                                    float* __restrict__ C, int M, int N, int K, int full,
+                                                                    int S, float* __restrict__ ws,
+                                                                    unsigned* __restrict__ cnt) {
+    sgemm_pieces<2>(A, B, C, M, N, K, full, S, ws, cnt);
+}
+extern "C" __global__ void __launch_bounds__(512) sgpu_sgemm_pieces_wide(const float* __restrict__ A,
+                                                                         const float* __restrict__ B, float* __restrict__ C,
+                                                                         int M, int N, int K, int full, int S,
+                                                                         float* __restrict__ ws,
+                                                                         unsigned* __restrict__ cnt) {
+    sgemm_pieces<4>(A, B, C, M, N, K, full, S, ws, cnt);
+}

@@ -815,6 +815,86 @@ def test_opt_unaligned_kwave128_shape_takes_the_size_rule_member(gpu):
     assert np.array_equal(C, D)
 
 
+# sgpu_sgemm_pieces: tiles of 128x128 and 128x256 that end at M and N, k-slices of 32 with a last one
+# that overlaps, tails split over K (few tiles, or more tiles than CUs), odd float alignments.
+PIECES_CASES = [(128, 128, 32), (129, 128, 33), (128, 255, 63), (300, 257, 100), (255, 513, 31 * 32 + 1),
+                (640, 384, 4097), (2047, 2049, 130), (1100, 8200, 65), (2049, 4111, 200)]
+
+
+@pytest.mark.parametrize("a_off,b_off", [(0, 0), (1, 3)])
+@pytest.mark.parametrize("M,N,K", PIECES_CASES)
+def test_pieces_integer_exact(gpu, M, N, K, a_off, b_off):
+    """Integers of 20 bits times small integers: exact only if all three pieces take part."""
+    say(f"sgemm pieces integer {M}x{N}x{K} a_off={a_off}")
+    rng = np.random.default_rng(M + N + K)
+    big = min(1 << 20, (1 << 24) // (2 * K))
+    A = rng.integers(-big, big + 1, (M, K)).astype(np.float32)
+    B = rng.integers(-2, 3, (K, N)).astype(np.float32)
+    want = (A.astype(np.float64) @ B.astype(np.float64)).astype(np.float32)
+    for _ in range(2):
+        assert np.array_equal(run_sgemm(gpu, "sgpu_sgemm_pieces", A, B, M, N, K, a_off, b_off), want)
+
+
+@pytest.mark.parametrize("scale_a,scale_b", [(1.0, 1.0), (1e-36, 1.0), (1.0, 1e-38), (1e-20, 1e-18), (1e30, 1e-30),
+                                             (3e38, 1e-3)])
+def test_pieces_scales(gpu, scale_a, scale_b):
+    """Results as close to float64 as fp32 sums are (64 random signs a sum: within 1e-6 of the
+    norm) for magnitudes that the cut keeps whole and for those where it would not: rows or
+    columns of tiny numbers, tiny products, numbers that round up to infinity as bf16.  Where the
+    result itself is subnormal (1e-38), to the subnormals' own spacing."""
+    M, N, K = 200, 300, 64
+    rng = np.random.default_rng(9)
+    A = (rng.uniform(0.5, 1.0, (M, K)) * rng.choice([-1, 1], (M, K)) * scale_a).astype(np.float32)
+    B = (rng.uniform(0.5, 1.0, (K, N)) * rng.choice([-1, 1], (K, N)) * scale_b).astype(np.float32)
+    if scale_a > 1e38:
+        A[3, 5] = np.float32(3.4028e38)
+    got = run_sgemm(gpu, "sgpu_sgemm_pieces", A, B, M, N, K).astype(np.float64)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    assert np.isfinite(got).all()
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want) + 64 * 2.0**-149 * np.sqrt(M * N)
+
+
+@pytest.mark.parametrize("M,N,K", [(128, 128, 64), (300, 257, 100), (2047, 2049, 130)])
+def test_pieces_nonfinite_and_nan_padding(gpu, M, N, K):
+    """Non-finite operands as IEEE fp32 has them, a row of A of zeros, and operands that are
+    followed by NaN: no load passes their ends."""
+    A, B, want = nonfinite_operands(M, N, K, M + N)
+    ha, hb = np.full(M * K + 512, np.nan, np.float32), np.full((K + 64) * N, np.nan, np.float32)
+    ha[:M * K], hb[:K * N] = A.reshape(-1), B.reshape(-1)
+    dA, dB, dC = gpu.DeviceArray.from_host(ha), gpu.DeviceArray.from_host(hb), gpu.DeviceArray((M, N))
+    dC.fill_bytes(0xFF)
+    gpu.call("sgpu_sgemm_pieces", dA.ptr, dB.ptr, dC.ptr, M, N, K, None)
+    gpu.synchronize()
+    assert np.array_equal(dC.to_host(), want, equal_nan=True)
+
+
+def test_pieces_graph_replay_and_refused_shapes(gpu):
+    """Recorded on a stream without a workspace (tail unsplit) and replayed with other inputs; and
+    sizes and alignments it does not take."""
+    M, N, K = 300, 700, 520
+    dA, dB, dC = gpu.DeviceArray((M, K)), gpu.DeviceArray((K, N)), gpu.DeviceArray((M, N))
+    st = gpu.Stream()
+    with gpu.Graph(st) as g:
+        gpu.call("sgpu_sgemm_pieces", dA.ptr, dB.ptr, dC.ptr, M, N, K, st.h)
+    for rep in range(3):
+        rng = np.random.default_rng(rep)
+        A, B = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N)).astype(np.float32)
+        gpu.call("sgpu_memcpy_htod", dA.ptr, A.ctypes.data, A.nbytes)
+        gpu.call("sgpu_memcpy_htod", dB.ptr, B.ctypes.data, B.nbytes)
+        dC.fill_bytes(0xFF)
+        g.launch()
+        st.synchronize()
+        ref = A.astype(np.float64) @ B.astype(np.float64)
+        assert np.abs(dC.to_host() - ref).max() / np.abs(ref).max() <= 1e-6
+    g.close()
+    st.close()
+    L = gpu.lib()
+    for m, n, k in ((127, 128, 32), (128, 127, 32), (128, 128, 31), (-1, 128, 32)):
+        assert L.sgpu_sgemm_pieces(dA.ptr, dB.ptr, dC.ptr, m, n, k, None) == gpu.SGPU_ERR_INVALID_ARG
+    assert L.sgpu_sgemm_pieces(dA.ptr + 2, dB.ptr, dC.ptr, 128, 128, 32, None) == gpu.SGPU_ERR_INVALID_ARG
+    assert L.sgpu_sgemm_pieces(dA.ptr, dB.ptr, dC.ptr, 0, 128, 32, None) == 0
+
+
 @pytest.mark.parametrize("tile", [16, 32])
 def test_small_reference_generator_unaligned_and_k_zero(gpu, og, tile):
     """Reference-generator inputs within the normwise bar of the oracle with A one float past

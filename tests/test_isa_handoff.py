@@ -31,6 +31,8 @@ KERNELS = [
     ("sgpu_decode", "sgpu_pf_gemm"),             # the Qwen prefill's split GEMM
     ("sgpu_prefill", "sgpu_pf_mm_22"),           # the prompt products in fp16 pieces, split
     ("sgpu_prefill", "sgpu_pf_mm_11"),
+    ("sgpu_pieces", "sgpu_sgemm_pieces"),        # the bf16-piece SGEMM's split tail
+    ("sgpu_pieces", "sgpu_sgemm_pieces_wide"),
     ("sgpu_decode", "sgpu_dec_attn32"),          # decode attention, chunked caches
     ("sgpu_decode", "sgpu_dec_attn64"),
     ("sgpu_decode", "sgpu_dec_attn128"),
