@@ -227,23 +227,35 @@ __device__ __forceinline__ void sgemm_pieces(const float* __restrict__ A, const 
         }
         __syncthreads();
         if (!last_s) return;
+        // all parts in order, this block's own among them; a tile's (narrow: two tiles') loads are
+        // issued before the first add
+        constexpr int U = 4 / NJ;
         float big = 0.0f;
-        for (int s2 = 0; s2 < S; s2++) {                   // all parts in order, this block's own among them
-            const float* src = ws + (size_t)(s2 * rest + part) * REC;
+        for (int s2 = 0; s2 < S; s2 += U) {
+            f32x4 v[U][4][NJ];
+            float m[U];
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                f32x4 v[NJ];
+            for (int u = 0; u < U; u++) {
+                const float* src = ws + (size_t)(min(s2 + u, S - 1) * rest + part) * REC;
 #pragma unroll
-                for (int j = 0; j < NJ; j++)
+                for (int i = 0; i < 4; i++)
 #pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        v[j][e] = __hip_atomic_load(src + ((i * NJ + j) * 4 + e) * 512 + tid, __ATOMIC_RELAXED,
-                                                    __HIP_MEMORY_SCOPE_AGENT);
+                    for (int j = 0; j < NJ; j++)
 #pragma unroll
-                for (int j = 0; j < NJ; j++) acc[i][j] = s2 == 0 ? v[j] : acc[i][j] + v[j];
+                        for (int e = 0; e < 4; e++)
+                            v[u][i][j][e] = __hip_atomic_load(src + ((i * NJ + j) * 4 + e) * 512 + tid, __ATOMIC_RELAXED,
+                                                              __HIP_MEMORY_SCOPE_AGENT);
+                m[u] = tid < TM + TN ? __hip_atomic_load(src + TM * TN + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0f;
             }
-            if (tid < TM + TN)
-                big = fmaxf(big, __hip_atomic_load(src + TM * TN + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (s2 + u >= S) break;
+                big = fmaxf(big, m[u]);
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) acc[i][j] = s2 + u == 0 ? v[u][i][j] : acc[i][j] + v[u][i][j];
+            }
         }
         if (tid < TM + TN) rmax[tid] = big;
         if (tid == 0) __hip_atomic_store(cnt + part, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
