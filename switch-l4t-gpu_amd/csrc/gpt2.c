@@ -74,6 +74,7 @@ struct sgpu_gpt2 {
     float *xT, *ln1T, *qkvT, *attT, *yT, *ln2T, *fcT;     /* batched prefill */
     float *d_q;                                     /* q of the fused path */
     int *d_step;                                    /* {token, pos} read by the fused kernels */
+    int *d_pf_ids;                                  /* prompt ids */
     int *d_tokens;                                  /* CTX + 1 greedy ids, by position */
     float *d_amax_v;                                /* argmax partials */
     int *d_amax_i;
@@ -100,6 +101,7 @@ void sgpu_gpt2_destroy(sgpu_gpt2 *e) {
     for (size_t i = 0; i < sizeof bufs / sizeof bufs[0]; i++) sgpu_free(bufs[i]);
     sgpu_free(e->d_step);
     sgpu_free(e->d_tokens);
+    sgpu_free(e->d_pf_ids);
     sgpu_free(e->d_amax_i);
     sgpu_free(e->d_attn_cnt);
     sgpu_free(e->d_split_cnt);
@@ -153,6 +155,7 @@ int sgpu_gpt2_create(sgpu_gpt2 **out, const sgpu_gpt2_cfg *c, const float *blob)
     TRY(sgpu_malloc((void **)&e->d_step, 4 * sizeof(int)));
     TRY(sgpu_memset_d8(e->d_step, 0, 4 * sizeof(int)));
     TRY(sgpu_malloc((void **)&e->d_tokens, (CTX + 1) * sizeof(int)));
+    TRY(sgpu_malloc((void **)&e->d_pf_ids, CTX * sizeof(int)));
     TRY(zalloc(&e->d_attn_ws, SGPU_ATTN_WS_FLOATS(c->NH, c->HD)));
     TRY(sgpu_malloc((void **)&e->d_attn_cnt, (size_t)c->NH * sizeof(unsigned)));
     TRY(sgpu_memset_d8(e->d_attn_cnt, 0, (size_t)c->NH * sizeof(unsigned)));
@@ -371,9 +374,8 @@ int sgpu_gpt2_forward_stages(sgpu_gpt2 *e, int token, int pos, float *logits_hos
 
 /* gpu_prefill's layer loop: all T prompt rows through each layer, cache positions 0..T-1
  * filled, the final rows left in xT.  Attention: the reference's per-row launches (k/v copies,
- * scores, softmax, mix for each row), or -- with the cache within 8192 positions -- two
- * strided copies of every row's k and v into the caches and one launch of the batched causal
- * attention. */
+ * scores, softmax, mix for each row), or -- with the cache within 8192 positions -- one
+ * launch for every row's k and v into the caches and one of the batched causal attention. */
 static int prefill_layers(sgpu_gpt2 *e, const int *ids, int T) {
     const sgpu_gpt2_cfg *c = &e->cfg;
     const int C = c->C, FC = c->FC;
@@ -382,21 +384,16 @@ static int prefill_layers(sgpu_gpt2 *e, const int *ids, int T) {
     const float *W = e->w;
     int rc;
 #define TRY(x) do { if ((rc = (x))) return rc; } while (0)
-    for (int t = 0; t < T; t++)
-        TRY(sgpu_add2(W + e->L.wte + (size_t)ids[t] * C, W + e->L.wpe + (size_t)t * C, e->xT + (size_t)t * C, C, s));
+    hipError_t hc = hipMemcpyAsync(e->d_pf_ids, ids, (size_t)T * sizeof(int), hipMemcpyHostToDevice, e->stream);
+    if (hc != hipSuccess) return (int)hc;
+    TRY(sgpu_internal_pf_g2embed(W + e->L.wte, W + e->L.wpe, e->d_pf_ids, T, e->xT, C, s));
     for (int l = 0; l < c->NL; l++) {
         const float *b = W + e->L.l_base + (size_t)l * e->L.lstride;
         TRY(sgpu_layernorm(e->xT, b + e->L.ln1w, b + e->L.ln1b, e->ln1T, C, eps, T, s));
         TRY(sgpu_internal_gemv_multi(b + e->L.qkvw, e->ln1T, b + e->L.qkvb, e->qkvT, C, 3 * C, T,
             e->d_split_ws, e->d_split_cnt, s));
         if (T <= 8192) {
-            const size_t row = (size_t)C * 4, qrow = 3 * row;
-            hipError_t he = hipMemcpy2DAsync(e->kc[l], row, e->qkvT + C, qrow, row, (size_t)T, hipMemcpyDeviceToDevice,
-                                             e->stream);
-            if (he == hipSuccess)
-                he = hipMemcpy2DAsync(e->vc[l], row, e->qkvT + 2 * C, qrow, row, (size_t)T, hipMemcpyDeviceToDevice,
-                                      e->stream);
-            if (he != hipSuccess) return (int)he;
+            TRY(sgpu_internal_pf_g2kv(e->qkvT, T, e->kc[l], e->vc[l], C, s));
             TRY(sgpu_internal_pf_attn(e->qkvT, e->kc[l], e->vc[l], e->attT, NULL, NULL, T, 0, c->NH, c->NH, c->HD, scale, s));
         } else {
             for (int t = 0; t < T; t++) {     /* causal attention, one query row at a time */

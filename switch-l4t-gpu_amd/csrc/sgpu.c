@@ -119,7 +119,7 @@ typedef struct {
     hipFunction_t dec_attn[3], dec_embed, dec_argmax_part, dec_argmax_embed;
     hipFunction_t dec_g2embed, dec_argmax_g2embed;
     hipFunction_t pf_embed, pf_gemm, pf_qkv_post, pf_attn[3], pf_swiglu;
-    hipFunction_t pf_mm[NPFMM], pf_gateup, pf_rms, h16_flush;
+    hipFunction_t pf_mm[NPFMM], pf_gateup, pf_rms, h16_flush, pf_g2embed, pf_g2kv;
     /* Split-K workspaces, one per stream that has launched split work (slot 0: the null
      * stream, made with the device state): partial tiles (SK_WS_FLOATS) and arrival counters
      * (SK_MAX_TILES, zero between launches).  Launches on one stream run in order, so a
@@ -241,6 +241,8 @@ static int load_device(int dev) {
             hipModuleGetFunction(&d->pf_qkv_post, d->mod[MOD_DECODE], "sgpu_pf_qkv_post") != hipSuccess ||
             hipModuleGetFunction(&d->pf_swiglu, d->mod[MOD_DECODE], "sgpu_pf_swiglu") != hipSuccess ||
             hipModuleGetFunction(&d->pf_gateup, d->mod[MOD_PREFILL], "sgpu_pf_gateup") != hipSuccess ||
+            hipModuleGetFunction(&d->pf_g2embed, d->mod[MOD_DECODE], "sgpu_pf_g2embed") != hipSuccess ||
+            hipModuleGetFunction(&d->pf_g2kv, d->mod[MOD_DECODE], "sgpu_pf_g2kv") != hipSuccess ||
             hipModuleGetFunction(&d->pf_rms, d->mod[MOD_PREFILL], "sgpu_pf_rms") != hipSuccess ||
             hipModuleGetFunction(&d->h16_flush, d->mod[MOD_PREFILL], "sgpu_h16_flush") != hipSuccess) {
             rc = SGPU_ERR_NO_KERNEL;
@@ -1714,6 +1716,26 @@ int sgpu_internal_pf_embed(const uint16_t *emb, const int *ids, int T, float *x,
     unsigned g[3] = {(unsigned)elem_grid((int)umin((unsigned)((long long)T * C), 0x7fffffffu)), 1, 1}, b[3] = {256, 1, 1};
     void *args[] = {(void *)&emb, (void *)&ids, &T, (void *)&x, &C};
     return launch(d->pf_embed, g, b, stream, args);
+}
+
+int sgpu_internal_pf_g2embed(const float *wte, const float *wpe, const int *ids, int T, float *x, int C, void *stream) {
+    if (!wte || !wpe || !ids || !x || T <= 0 || C <= 0 || C % 4) return SGPU_ERR_INVALID_ARG;
+    int rc;
+    devstate *d = cur(&rc);
+    if (!d) return rc;
+    unsigned g[3] = {umin(cdiv((long long)T * (C / 4), 256), 65535u), 1, 1}, b[3] = {256, 1, 1};
+    void *args[] = {(void *)&wte, (void *)&wpe, (void *)&ids, &T, (void *)&x, &C};
+    return launch(d->pf_g2embed, g, b, stream, args);
+}
+
+int sgpu_internal_pf_g2kv(const float *qkv, int T, float *kc, float *vc, int C, void *stream) {
+    if (!qkv || !kc || !vc || T <= 0 || C <= 0 || C % 4) return SGPU_ERR_INVALID_ARG;
+    int rc;
+    devstate *d = cur(&rc);
+    if (!d) return rc;
+    unsigned g[3] = {umin(cdiv((long long)T * (C / 2), 256), 65535u), 1, 1}, b[3] = {256, 1, 1};
+    void *args[] = {(void *)&qkv, &T, (void *)&kc, (void *)&vc, &C};
+    return launch(d->pf_g2kv, g, b, stream, args);
 }
 
 int sgpu_internal_pf_gemm(const uint16_t *W, const float *X, const float *bias, float *Y, int K, int N, int T,

@@ -455,6 +455,35 @@ __global__ void sgpu_pf_embed(const uint16_t* __restrict__ emb, const int* __res
     }
 }
 
+// GPT-2: x[t] = wte[ids[t]] + wpe[t] for the T rows (C % 4 == 0), the additions of
+// gpt2_engine.c:176-179.  Bound by launch latency: one launch took the place of one per row, 0.56 ms
+// of a 300-row prompt's 3.4.
+__global__ void __launch_bounds__(256) sgpu_pf_g2embed(const float* __restrict__ wte, const float* __restrict__ wpe,
+                                                       const int* __restrict__ ids, int T, float* __restrict__ x, int C) {
+#pragma clang fp contract(off)
+    const int q = C / 4;
+    const long long total = (long long)T * q;
+    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < total; i += (long long)gridDim.x * blockDim.x) {
+        const int t = (int)(i / q), k = 4 * (int)(i % q);
+        const sgpu_f32x4 a = *reinterpret_cast<const sgpu_f32x4_a4*>(wte + (size_t)ids[t] * C + k);
+        const sgpu_f32x4 b = *reinterpret_cast<const sgpu_f32x4_a4*>(wpe + (size_t)t * C + k);
+        *reinterpret_cast<sgpu_f32x4_a4*>(x + (size_t)t * C + k) = a + b;
+    }
+}
+
+// GPT-2: rows C..2C-1 and 2C..3C-1 of each prompt row's qkv vector into the key and value cache
+// (C % 4 == 0).
+__global__ void __launch_bounds__(256) sgpu_pf_g2kv(const float* __restrict__ qkv, int T, float* __restrict__ kc,
+                                                    float* __restrict__ vc, int C) {
+    const int q = C / 2;
+    const long long total = (long long)T * q;
+    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < total; i += (long long)gridDim.x * blockDim.x) {
+        const int t = (int)(i / q), k = 4 * (int)(i % q);
+        const sgpu_f32x4 v = *reinterpret_cast<const sgpu_f32x4_a4*>(qkv + (size_t)t * 3 * C + C + k);
+        *reinterpret_cast<sgpu_f32x4_a4*>((k < C ? kc + k : vc + (k - C)) + (size_t)t * C) = v;
+    }
+}
+
 // Y[t][n] = sum_k X[t][k] * h2f(W[n][k]) + bias?[n] on the fp32 matrix cores (one block per
 // 32-token x 32-row tile and k-split, grid-stride over units; blockDim 256, K % 4 == 0,
 // 16-byte X rows).  S > 1 splits each tile's K over S blocks (ws: S * tiles * 1024 floats,

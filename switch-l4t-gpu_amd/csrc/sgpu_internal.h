@@ -49,6 +49,11 @@ SGPU_HIDDEN int sgpu_internal_dec_argmax_next(const float *v, int n, float *part
  * of k into the key cache with v into the value cache, causal attention of T prompt rows
  * (positions pos0..pos0+T-1, pos0 + T <= 8192), and row SwiGLU over gate|up rows of 2*FC. */
 SGPU_HIDDEN int sgpu_internal_pf_embed(const uint16_t *emb, const int *ids, int T, float *x, int C, void *stream);
+/* GPT-2's prompt rows wte[ids[t]] + wpe[t], and their k and v (of qkv rows of 3*C) into the caches;
+ * C % 4 == 0. */
+SGPU_HIDDEN int sgpu_internal_pf_g2embed(const float *wte, const float *wpe, const int *ids, int T, float *x, int C,
+                                         void *stream);
+SGPU_HIDDEN int sgpu_internal_pf_g2kv(const float *qkv, int T, float *kc, float *vc, int C, void *stream);
 /* accum != 0: Y += X W^T (+ bias), the residual add fused into the GEMM. */
 SGPU_HIDDEN int sgpu_internal_pf_gemm(const uint16_t *W, const float *X, const float *bias, float *Y, int K, int N,
                                       int T, float *ws, unsigned *cnt, int accum, void *stream);
