@@ -14,7 +14,7 @@
 // chosen over the finite ones.
 //
 // Measured against the same layers on fp32 MFMA tiles (sgpu_pf_gemm, 32x32 per block): a prompt
-// of 500 rows of the Qwen2.5-0.5B sizes 6.08 -> 3.35 ms, of 3001 rows 39.5 -> 12.1 ms; distance
+// of 500 rows of the Qwen2.5-0.5B sizes 6.08 -> 3.30 ms, of 3001 rows 39.5 -> 11.5 ms; distance
 // of the logits from a 64-bit forward 1.1e-6 -> 6.4e-7 and 9.3e-7 -> 8.0e-7.
 //
 // This code object keeps fp16 subnormals (the pieces use them).  The reference reads subnormal
@@ -361,8 +361,9 @@ __device__ __forceinline__ void pf_mm(const uint16_t* __restrict__ W, const uint
 // running maximum, sum and output over its tiles (online softmax) and the four are merged once
 // through LDS at the end, so the key loop has no barrier and a short prompt still fills the
 // CUs' SIMDs.  Both products are laid out so that no operand passes through LDS:
-//  * scores transposed, S^T = K Q^T: lane (l32, h) feeds key l32's dims HD/2*h.. as A and query
-//    l32's as B (16-byte loads; the k order of a dot product is free), so accumulator r of a
+//  * scores transposed, S^T = K Q^T: lane (l32, h) feeds key l32's dims 8*v + 4*h.. as A and query
+//    l32's as B (16-byte loads, the halves' side by side; the k order of a dot product is free:
+//    with dims HD/2*h.. each load touched twice the cache lines), so accumulator r of a
 //    lane is key 8*(r/4) + 4*h + r%4 of query l32 and the softmax over keys is in-lane, plus
 //    one exchange between the lane halves;
 //  * O^T = V^T P^T: step r multiplies the keys the lanes hold in accumulator r, so P is the B
@@ -372,9 +373,8 @@ __device__ __forceinline__ void pf_mm(const uint16_t* __restrict__ W, const uint
 // Loads go through buffer resources that end at the last valid key row: rows past it read as
 // zero and are masked.  The heavy blocks (last rows) are dispatched first.
 // Measured against one block per head and row on the vector ALUs, which read K and V once per
-// row: 50 -> 17 us a launch at 500 rows, 14 query and 2 KV heads of 64 (the whole prompt 6.89 ->
-// 6.08 ms); a 3001-row prompt in chunks of 512 rows 232 -> 41 us a launch on average (67.1 ->
-// 39.5 ms).
+// row, 14 query and 2 KV heads of 64: 50 -> 16 us a launch at 500 rows, 1390 -> 172 us for 3001 rows
+// (194 with expf and with a lane's dims of K in one run).
 template <int HD>
 __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const float* __restrict__ kc,
                                         const float* __restrict__ vc, float* __restrict__ out, uint16_t* __restrict__ P,
@@ -393,17 +393,17 @@ __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const flo
 
     float qv[HH];
     {
-        const float* qr = qkv + (size_t)min(q0 + l32, T - 1) * QKVD + (size_t)head * HD + HH * h;
+        const float* qr = qkv + (size_t)min(q0 + l32, T - 1) * QKVD + (size_t)head * HD + 4 * h;
 #pragma unroll
         for (int v = 0; v < HH / 4; v++) {
-            const sgpu_f32x4 a = *reinterpret_cast<const sgpu_f32x4*>(qr + 4 * v);
+            const sgpu_f32x4 a = *reinterpret_cast<const sgpu_f32x4*>(qr + 8 * v);
 #pragma unroll
             for (int e = 0; e < 4; e++) qv[4 * v + e] = a[e];
         }
     }
     sgpu_f32x4 kr[HH / 4];
     vseg vr[16];
-    const int koff = (l32 * KVD + HH * h) * 4, voff = (4 * h * KVD + NB * l32) * 4;
+    const int koff = (l32 * KVD + 4 * h) * 4, voff = (4 * h * KVD + NB * l32) * 4;
     auto tile_rsrc = [&](const float* c, int t) __attribute__((always_inline)) {
         const int rows = max(n - 32 * t, 0);
         return __builtin_amdgcn_make_buffer_rsrc((void*)(c + (size_t)g * HD + (size_t)t * 32 * KVD), (short)0,
@@ -413,7 +413,7 @@ __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const flo
         const __amdgpu_buffer_rsrc_t rs = tile_rsrc(kc, t);
 #pragma unroll
         for (int v = 0; v < HH / 4; v++)
-            kr[v] = __builtin_bit_cast(sgpu_f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, koff + 16 * v, 0, 0));
+            kr[v] = __builtin_bit_cast(sgpu_f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, koff + 32 * v, 0, 0));
     };
     auto load_v = [&](int t) __attribute__((always_inline)) {
         const __amdgpu_buffer_rsrc_t rs = tile_rsrc(vc, t);
@@ -426,6 +426,8 @@ __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const flo
         }
     };
 
+    // The softmax in powers of two: scores carry log2(e), so a weight is one v_exp_f32.
+    const float scale2 = scale * 1.44269504088896340736f;
     f32x16 o[NB];
 #pragma unroll
     for (int j = 0; j < NB; j++)
@@ -446,7 +448,7 @@ __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const flo
         load_k(t + 4);
         float mx = -INFINITY;
 #pragma unroll
-        for (int r = 0; r < 16; r++) s[r] = (s[r] + s1[r]) * scale;
+        for (int r = 0; r < 16; r++) s[r] = (s[r] + s1[r]) * scale2;
         if (32 * t + 31 > pos0 + q0) {                // the tile reaches past some row's own position
 #pragma unroll
             for (int r = 0; r < 16; r++)
@@ -456,12 +458,12 @@ __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const flo
         for (int r = 0; r < 16; r++) mx = fmaxf(mx, s[r]);
         mx = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32)));
         const float base = mx == -INFINITY ? 0.0f : mx;   // every key so far masked: weights are all zero
-        const float al = expf(m - base);
+        const float al = __builtin_amdgcn_exp2f(m - base);
         m = mx;
         float sum = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-            s[r] = expf(s[r] - base);
+            s[r] = __builtin_amdgcn_exp2f(s[r] - base);
             sum += s[r];
         }
         l = l * al + sum;
@@ -498,7 +500,7 @@ __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const flo
     float wt[4], L = 0.0f;
 #pragma unroll
     for (int w = 0; w < 4; w++) {
-        wt[w] = expf(ml[w][0][q] - M);
+        wt[w] = __builtin_amdgcn_exp2f(ml[w][0][q] - M);
         L = __builtin_fmaf(ml[w][1][q], wt[w], L);
     }
     float v[HD / 8];
@@ -570,8 +572,13 @@ __global__ void __launch_bounds__(256) sgpu_pf_rms(const float* __restrict__ x, 
     x += t * n;
     P += t * 3 * n;
     pd += t * (n / G);
-    float local = 0.0f;
-    for (int k = 4 * tid; k < n; k += 1024) {
+    // the thread's first four values and gains stay in registers, both loaded before the reduction
+    typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+    const int k4 = min(4 * tid, n - 4);
+    const sgpu_f32x4 x4 = *reinterpret_cast<const sgpu_f32x4*>(x + k4);
+    const u16x4 w4 = *reinterpret_cast<const u16x4*>(w + k4);
+    float local = 4 * tid < n ? (x4[0] * x4[0] + x4[1] * x4[1]) + (x4[2] * x4[2] + x4[3] * x4[3]) : 0.0f;
+    for (int k = 4 * tid + 1024; k < n; k += 1024) {
         const sgpu_f32x4 v = *reinterpret_cast<const sgpu_f32x4*>(x + k);
         local += (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
     }
@@ -586,10 +593,11 @@ __global__ void __launch_bounds__(256) sgpu_pf_rms(const float* __restrict__ x, 
         float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
         uint32_t m = 0;
         if (ok) {
-            const sgpu_f32x4 v = *reinterpret_cast<const sgpu_f32x4*>(x + k);
+            const sgpu_f32x4 v = k0 == 0 ? x4 : *reinterpret_cast<const sgpu_f32x4*>(x + k);
+            const u16x4 g = k0 == 0 ? w4 : *reinterpret_cast<const u16x4*>(w + k);
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                y[e] = v[e] * inv * sgpu_h2f(w[k + e]);
+                y[e] = v[e] * inv * sgpu_h2f(g[e]);
                 m = max(m, mag_bits(y[e]));
             }
         }
