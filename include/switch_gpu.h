@@ -157,6 +157,9 @@ int sgpu_sgemm_opt(const float *A, const float *B, float *C, int M, int N, int K
  * kernels of these names are the fp32 members themselves.
  * No counterpart in the reference (its sgemm_opt is one kernel). */
 const char *sgpu_sgemm_opt_plan(int M, int N, int K, int cus, int *splits);
+/* The kernel of the piece form when sgpu_sgemm_opt takes it (a workspace at hand), else NULL;
+ * a pure function. */
+const char *sgpu_sgemm_opt_pieces(int M, int N, int K, int cus);
 /* The sgemm_opt256 member alone (any shape; masked loads on edge tiles).  No
  * counterpart in the reference: an added member of the same family, with the same
  * (A, B, C, M, N, K) symbol arguments, for hosts that launch members by name. */

@@ -518,7 +518,7 @@ int sgpu_qwen_phase_times(sgpu_qwen *e, int pos, int reps, float *us) {
  *    to MM_MIN_ROWS rows and for head or layer sizes that are no whole 64-blocks. ---- */
 #define PF_ROWS 512
 #define MM_ROWS 4096
-#define MM_MIN_ROWS 64
+#define MM_MIN_ROWS 64       /* about where they meet: 77 us a layer on fp32 tiles at 64 rows, some 80 in pieces */
 
 static int mm_ok(const sgpu_qwen_cfg *c) {
     const long long wide = c->FC > c->C ? c->FC : c->C;

@@ -796,7 +796,7 @@ static int pieces_launch(devstate *d, const float *A, const float *B, float *C, 
  * against the fp32 members' (rounds of 64x64 tiles at 14.3 ns per k, or the whole at 125 TFLOP/s).
  * Measured over 70 shapes of 64 to 8192 a side (log-uniform, K from 86 on) the rule's choices take
  * 14% less time than the fp32 members alone, the best choices 15% less; 4096^3 936 -> 602 us,
- * 3072^3 419 -> 270, 2048^3 121.6 -> 90.1, 4097^3 1102 -> 678, 2047x2049x2048 134.9 -> 117.7.
+ * 3072^3 419 -> 270, 2048^3 121.6 -> 90.1, 4097^3 1102 -> 678, 2047x2049x2048 134.9 -> 115.6.
  * Where it loses, the rule keeps the members: 1024^3 25.2 against 19.8, 1023x1025x997 25.4 against
  * 21.1, 3000x3000x128 35.7 against 27.3. */
 static int pieces_win(const pieces_plan *p, int M, int N, int K, int cus) {
@@ -1086,6 +1086,19 @@ const char *sgpu_sgemm_opt_plan(int M, int N, int K, int cus, int *splits) {
     return g_sgemm_members[p].name;
 }
 
+/* The plans whose product may run in its piece form. */
+static int plan_large(int p) {
+    if (p >= 0) return g_sgemm_members[p].kid == K_SGEMM_OPT || g_sgemm_members[p].kid == K_SGEMM_OPT256;
+    return p == PLAN_KWAVE128 || p == PLAN_KWAVE || p == PLAN_KWAVE_EDGE;
+}
+const char *sgpu_sgemm_opt_pieces(int M, int N, int K, int cus) {
+    int S;
+    if (M < 1 || N < 1 || K < 0 || cus < 1 || !pieces_shape(M, N, K) || !plan_large(opt_plan(M, N, K, cus, &S))) return NULL;
+    const pieces_plan p = pieces_best(M, N, K, cus, 1);
+    if (!pieces_win(&p, M, N, K, cus)) return NULL;
+    return p.wide ? "sgpu_sgemm_pieces_wide" : "sgpu_sgemm_pieces";
+}
+
 int sgpu_sgemm_opt(const float *A, const float *B, float *C, int M, int N, int K, void *stream) {
     if (M < 0 || N < 0 || K < 0) return SGPU_ERR_INVALID_ARG;
     if (M == 0 || N == 0) return SGPU_OK;
@@ -1100,9 +1113,7 @@ int sgpu_sgemm_opt(const float *A, const float *B, float *C, int M, int N, int K
     unsigned *cnt;
     if (p == PLAN_SPLITK && sk_workspace(d, stream, &ws, &cnt) == SGPU_OK)    /* else: the unsplit member */
         return splitk_launch(d, A, B, C, M, N, K, S, ws, cnt, stream);
-    const int big = p >= 0 && (g_sgemm_members[p].kid == K_SGEMM_OPT || g_sgemm_members[p].kid == K_SGEMM_OPT256);
-    if ((p == PLAN_KWAVE128 || p == PLAN_KWAVE || p == PLAN_KWAVE_EDGE || big) && pieces_taken(A, B, C, M, N, K, stream, &rc))
-        return rc;
+    if (plan_large(p) && pieces_taken(A, B, C, M, N, K, stream, &rc)) return rc;
     if (p == PLAN_KWAVE128 && !(((uintptr_t)A | (uintptr_t)B) & 15))
         return sgemm_common(K_SGEMM_KWAVE128, "sgemm_kwave128", A, B, C, M, N, K, stream);
     if (p == PLAN_KWAVE && !(((uintptr_t)A | (uintptr_t)B) & 15)) return kwave_launch(0, A, B, C, M, N, K, stream);

@@ -324,7 +324,7 @@ __device__ __forceinline__ void pf_mm(const uint16_t* __restrict__ W, const uint
             block_scale(m, up, down);
             // through LDS (the wave's own 6 KB, free after the k loop) so that a row's 64 codes of
             // a piece leave as one 128-byte line: 8-byte stores straight from the accumulators
-            // made it 175 us instead of 171 at 3001 rows
+            // took 311 us instead of 299 at 3001 rows and K 1792 (172 either way at K 896)
             uint16_t* const st = xs + wave * (3 * 16 * G);
 #pragma unroll
             for (int j = 0; j < 4; j++) {

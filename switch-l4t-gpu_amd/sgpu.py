@@ -73,6 +73,7 @@ _SIGS = {
     "sgpu_sgemm_tiled": (_I, [_P, _P, _P, _I, _I, _I, _P]),
     "sgpu_sgemm_tiled4": (_I, [_P, _P, _P, _I, _I, _I, _P]),
     "sgpu_sgemm_opt": (_I, [_P, _P, _P, _I, _I, _I, _P]),
+    "sgpu_sgemm_opt_pieces": (ct.c_char_p, [_I, _I, _I, _I]),
     "sgpu_sgemm_opt_plan": (ct.c_char_p, [_I, _I, _I, _I, ct.POINTER(_I)]),
     "sgpu_sgemm_opt256": (_I, [_P, _P, _P, _I, _I, _I, _P]),
     "sgpu_sgemm_kwave": (_I, [_P, _P, _P, _I, _I, _I, _P]),

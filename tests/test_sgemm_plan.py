@@ -148,6 +148,17 @@ def test_plan_rejects():
     assert sgpu.lib().sgpu_sgemm_opt_plan(64, 64, 64, 256, None) is not None
 
 
+@pytest.mark.parametrize("M,N,K,kernel", [
+    (4096, 4096, 4096, "sgpu_sgemm_pieces_wide"), (3072, 3072, 3072, "sgpu_sgemm_pieces_wide"),
+    (2048, 2048, 2048, "sgpu_sgemm_pieces"), (2047, 2049, 2048, "sgpu_sgemm_pieces"),
+    (4097, 4097, 4097, "sgpu_sgemm_pieces_wide"), (1024, 1024, 1024, None), (1023, 1025, 997, None),
+    (3000, 3000, 128, None), (768, 768, 2048, None), (127, 8192, 8192, None), (256, 256, 256, None)])
+def test_piece_form_pinned_at_256_cus(M, N, K, kernel):
+    """Where sgpu_sgemm_opt takes the piece form: measured faster there, slower on the others."""
+    got = sgpu.lib().sgpu_sgemm_opt_pieces(M, N, K, 256)
+    assert (got.decode() if got else None) == kernel
+
+
 def test_bench_traffic_record_covers_the_4096_member():
     """bench.py reports the HBM traffic of the member sgpu_sgemm_opt launches at 4096^3 from
     profiles/traffic.json under "<member>_4096"; a plan change that moves 4096^3 to another
