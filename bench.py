@@ -44,6 +44,7 @@ import sgpu  # noqa: E402
 
 METRIC = "SGEMM TFLOPS @4096³ + GEMV GB/s (% of HBM peak); decode tok/s"
 PEAK_FP32_MATRIX_TFLOPS = 157.3      # MI355X dense fp32 matrix
+PIECES_NOTE = ": fp32 operands cut exactly into three bf16 pieces, fp32 accumulation"
 PEAK_PIECES_TFLOPS = 2500.0 / 6      # ... dense bf16 matrix over the six piece products of an fp32 product
 PEAK_HBM_GBPS = 8000.0               # MI355X HBM3E
 PROFILE_TRAFFIC = os.path.join(ROOT, "profiles", "traffic.json")
@@ -773,7 +774,7 @@ def main():
         "data": "synthetic",
         "config": {"workload": "SGEMM C=A*B M=N=K=4096 fp32 row-major, A,B from srand(42) "
                                "(rand()%2000-1000)/1000, alpha=1 beta=0, sgpu_sgemm_opt (launches the member "
-                               f"{member} at this shape)",
+                               f"{member} at this shape{PIECES_NOTE if pieces else ''})",
                    "M": n, "N": n, "K": n, "parallelism": "single GPU"},
         "roofline": {"bound": "mfma", "achieved": round(achieved, 3), "peak": round(peak, 1),
                      "unit": "TFLOP/s", "frac": round(achieved / peak, 4),
