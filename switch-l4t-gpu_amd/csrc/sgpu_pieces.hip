@@ -25,6 +25,11 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int TM = 128, KS = 32;                       // tile rows, k per step
 
+template <bool V>
+struct bool_c {
+    constexpr operator bool() const { return V; }
+};
+
 // The three pieces of two numbers, packed: the first rounded to nearest, then the upper halves of
 // what is left (16 bits at most), which one v_perm takes for two numbers.
 __device__ __forceinline__ void cut2(float x0, float x1, uint32_t (&p)[3]) {
@@ -55,9 +60,10 @@ __device__ __noinline__ float serial_dot(const float* __restrict__ a, const floa
 // Measured at 4096^3: 8 waves and 128x256 590-602 us, 128x128 691; 4 waves and 128x128 822; one LDS
 // buffer and two blocks of 4 waves a CU 672; the fp32 members 926.  With chunk order c ^ (row / 4 % 4),
 // which puts two of a read's rows on the same banks, 610 and 724.
-// A last row or column of tiles that would pass M or N ends at M or N (its overlap is computed
-// twice, alike), a last step that would pass K starts at K - 32 with the k already summed set to
-// zero: no load needs a bound.  Operands of any float alignment.
+// A last row or column of tiles that would pass M or N ends at M or N and is stored from its first
+// new row or column on: the tile before it owns the overlap (one of the two may be split over K and
+// the other not, whose sums round differently).  A last step that would pass K starts at K - 32 with
+// the k already summed set to zero: no load needs a bound.  Operands of any float alignment.
 // The first `full` tiles are one block each; those that are left, too few for a round of all CUs, are
 // split over S blocks of consecutive slices each, whose sums meet by the hand-off of
 // sgpu_device.h: ws holds one record of 128 * TN + 128 + TN floats per block (its tile, then its
@@ -81,7 +87,8 @@ __device__ __forceinline__ void sgemm_pieces(const float* __restrict__ A, const 
     const int u = (int)blockIdx.x - full, part = whole ? 0 : u % rest, sp = whole ? 0 : u / rest;
     const int tile = whole ? xcd * (full / 8) + min(xcd, full % 8) + blockIdx.x / 8 : full + part;
     const int band = tile / (8 * ntn), bm = min(8, ntm - 8 * band), in = tile - band * 8 * ntn;
-    const int m0 = min((8 * band + in % bm) * TM, M - TM), n0 = min((in / bm) * TN, N - TN);
+    const int mt = (8 * band + in % bm) * TM, nt = (in / bm) * TN;         // first row and column of its own
+    const int m0 = min(mt, M - TM), n0 = min(nt, N - TN);
 
     // A thread's part of a slice: A rows r and r + 64, k 4 q..; B rows k 4 q + i, columns NJ r...
     const int r = tid >> 3, q = tid & 7;
@@ -268,24 +275,36 @@ __device__ __forceinline__ void sgemm_pieces(const float* __restrict__ A, const 
     float cmax[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; j++) cmax[j] = rmax[TM + lc + j];
+    auto store = [&](auto shifted) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+        for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int lm = 64 * wm + 16 * i + 4 * quarter + e, m = m0 + lm;
-            const float ra = rmax[lm];
-            rowv v;
-            bool redo = false;
+            for (int e = 0; e < 4; e++) {
+                const int lm = 64 * wm + 16 * i + 4 * quarter + e, m = m0 + lm;
+                const float ra = rmax[lm];
+                if (shifted && m < mt) continue;
+                rowv v;
+                bool redo = false;
 #pragma unroll
-            for (int j = 0; j < NJ; j++) {
-                v[j] = acc[i][j][e];
-                redo |= !__builtin_isfinite(v[j]) || (fminf(fminf(ra, cmax[j]) * 0x1p100f, ra * cmax[j] * 0x1p96f) < 1.0f &&
-                                                      ra > 0.0f && cmax[j] > 0.0f);
+                for (int j = 0; j < NJ; j++) {
+                    v[j] = acc[i][j][e];
+                    redo |= !__builtin_isfinite(v[j]) || (fminf(fminf(ra, cmax[j]) * 0x1p100f, ra * cmax[j] * 0x1p96f) < 1.0f &&
+                                                          ra > 0.0f && cmax[j] > 0.0f);
+                }
+                if (redo)
+                    for (int j = 0; j < NJ; j++) v[j] = serial_dot(A + (size_t)m * K, B + n + j, K, N);
+                float* const c = C + (size_t)m * N + n;
+                if (!shifted || n >= nt) {
+                    *reinterpret_cast<rowv_a4*>(c) = v;
+                } else {
+#pragma unroll
+                    for (int j = 0; j < NJ; j++)
+                        if (n + j >= nt) c[j] = v[j];
+                }
             }
-            if (redo)
-                for (int j = 0; j < NJ; j++) v[j] = serial_dot(A + (size_t)m * K, B + n + j, K, N);
-            *reinterpret_cast<rowv_a4*>(C + (size_t)m * N + n) = v;
-        }
+    };
+    if (m0 == mt && n0 == nt) store(bool_c<false>{});
+    else store(bool_c<true>{});
 }
 
 }  // namespace

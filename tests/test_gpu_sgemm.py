@@ -835,6 +835,46 @@ def test_pieces_integer_exact(gpu, M, N, K, a_off, b_off):
         assert np.array_equal(run_sgemm(gpu, "sgpu_sgemm_pieces", A, B, M, N, K, a_off, b_off), want)
 
 
+@pytest.mark.parametrize("M,N,K", [(1024, 4097, 2048), (2049, 4111, 2000), (3073, 3073, 3073), (4097, 4097, 4097),
+                                   (1090, 5147, 1751)])
+def test_pieces_overlap_has_one_owner(gpu, M, N, K):
+    """Shapes whose last row or column of tiles is shifted back over its neighbour and where, on 256
+    compute units, one of the two is split over K and the other is not: the elements of the unsplit
+    tiles (of each tile's own rows and columns) equal bit for bit the product recorded on a stream
+    without a workspace, which splits no tile; the split ones differ from it somewhere."""
+    say(f"sgemm pieces overlap {M}x{N}x{K}")
+    cus = gpu.device_props().compute_units
+    kernel = gpu.lib().sgpu_sgemm_opt_pieces(M, N, K, cus)
+    assert kernel
+    tn = 256 if kernel.endswith(b"_wide") else 128
+    rng = np.random.default_rng(M + N + K)
+    A, B = rng.uniform(-1, 1, (M, K)).astype(np.float32), rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    dA, dB, dC = gpu.DeviceArray.from_host(A), gpu.DeviceArray.from_host(B), gpu.DeviceArray((M, N))
+    st = gpu.Stream()
+    with gpu.Graph(st) as g:
+        gpu.call("sgpu_sgemm_pieces", dA.ptr, dB.ptr, dC.ptr, M, N, K, st.h)
+    g.launch()
+    st.synchronize()
+    unsplit = dC.to_host()
+    g.close()
+    st.close()
+    # the kernel's tile order: bands of eight tile rows, column by column
+    ntm, ntn = -(-M // 128), -(-N // tn)
+    full = ntm * ntn // cus * cus
+    order = [(i, j) for b in range(0, ntm, 8) for j in range(ntn) for i in range(b, min(b + 8, ntm))]
+    own = np.zeros((M, N), bool)
+    for i, j in order[:full]:
+        own[128 * i:128 * (i + 1), tn * j:tn * (j + 1)] = True
+    assert 0 < full < ntm * ntn
+    for _ in range(3):
+        dC.fill_bytes(0xFF)
+        gpu.call("sgpu_sgemm_pieces", dA.ptr, dB.ptr, dC.ptr, M, N, K, None)
+        gpu.synchronize()
+        got = dC.to_host()
+        assert np.array_equal(got[own], unsplit[own])
+        assert not np.array_equal(got[~own], unsplit[~own])
+
+
 @pytest.mark.parametrize("scale_a,scale_b", [(1.0, 1.0), (1e-36, 1.0), (1.0, 1e-38), (1e-20, 1e-18), (1e30, 1e-30),
                                              (3e38, 1e-3)])
 def test_pieces_scales(gpu, scale_a, scale_b):
