@@ -151,10 +151,10 @@ int sgpu_sgemm_opt(const float *A, const float *B, float *C, int M, int N, int K
  * "sgemm_kwave_edge" and "sgemm_kwave128" the member the size rule picks, and with an operand
  * off 4 bytes "sgemm_kwave" or "sgemm_kwave_edge" becomes the 64x64-or-larger member the size
  * rule picks.
- * A product of "sgemm_opt", "sgemm_opt256", "sgemm_kwave", "sgemm_kwave_edge" or
- * "sgemm_kwave128" runs in the form of sgpu_sgemm_pieces where that is estimated to be faster
- * (large problems, float-aligned operands), here and in the members' own launchers alike; the
- * kernels of these names are the fp32 members themselves.
+ * Where the plan is "sgemm_opt", "sgemm_opt256", "sgemm_kwave", "sgemm_kwave_edge" or
+ * "sgemm_kwave128" and the form of sgpu_sgemm_pieces is estimated to be faster (large problems,
+ * float-aligned operands), sgpu_sgemm_opt launches that form instead (sgpu_sgemm_opt_pieces tells);
+ * the members' own launchers always launch the fp32 members.
  * No counterpart in the reference (its sgemm_opt is one kernel). */
 const char *sgpu_sgemm_opt_plan(int M, int N, int K, int cus, int *splits);
 /* The kernel of the piece form when sgpu_sgemm_opt takes it (a workspace at hand), else NULL;
@@ -205,7 +205,8 @@ int sgpu_sgemm_pieces(const float *A, const float *B, float *C, int M, int N, in
  * tile sums all S partials in split order, so results do not depend on arrival order.
  * Rejects problems needing more than 16384 tiles or S x tiles x 4096 floats (32 MB) of
  * workspace (SGPU_ERR_INVALID_ARG).  No counterpart in the reference.
- * Split-K workspaces (also used by sgpu_sgemm_opt and sgpu_gemv_multi when they split K): one
+ * Split-K workspaces (also used by sgpu_sgemm_opt, sgpu_sgemm_pieces and sgpu_gemv_multi when they
+ * split K or the last tiles' K): one
  * per stream, so launches on different streams or from different host threads may overlap;
  * launches on one stream run in order.  The null stream's is made by sgpu_init; another
  * stream's on its first launch that splits (32 MB + 64 KB, at most 32 streams per device),
@@ -214,7 +215,7 @@ int sgpu_sgemm_pieces(const float *A, const float *B, float *C, int M, int N, in
  * thread and gets none: sgpu_sgemm_splitk returns SGPU_ERR_NO_WORKSPACE on it.  A stream
  * being recorded (sgpu_graph_begin) cannot get one: make its first split launch before
  * recording, else sgpu_sgemm_splitk returns SGPU_ERR_NO_WORKSPACE; on either kind of stream
- * sgpu_sgemm_opt / sgpu_gemv_multi launch their unsplit kernels instead.  A recorded graph
+ * sgpu_sgemm_opt / sgpu_sgemm_pieces / sgpu_gemv_multi launch their unsplit kernels instead.  A recorded graph
  * uses the workspace of the stream it was recorded on, which stays allocated while the graph
  * exists, also after that stream is destroyed; do not replay the graph concurrently with
  * itself or with other split launches on that stream. */

@@ -706,10 +706,7 @@ int sgpu_sgemm_tiled(const float *A, const float *B, float *C, int M, int N, int
 int sgpu_sgemm_tiled4(const float *A, const float *B, float *C, int M, int N, int K, void *stream) {
     return sgemm_common(K_SGEMM_TILED4, "sgemm_tiled4", A, B, C, M, N, K, stream);
 }
-static int pieces_taken(const float *A, const float *B, float *C, int M, int N, int K, void *stream, int *rc);
 int sgpu_sgemm_opt256(const float *A, const float *B, float *C, int M, int N, int K, void *stream) {
-    int rc;
-    if (pieces_taken(A, B, C, M, N, K, stream, &rc)) return rc;
     return sgemm_common(K_SGEMM_OPT256, "sgemm_opt256", A, B, C, M, N, K, stream);
 }
 /* sgemm_kwave's problems: M, N multiples of 64, K a multiple of 32 (the operands' 16-byte
@@ -730,8 +727,6 @@ int sgpu_sgemm_kwave(const float *A, const float *B, float *C, int M, int N, int
     if (M < 0 || N < 0 || K < 0) return SGPU_ERR_INVALID_ARG;
     if (M == 0 || N == 0) return SGPU_OK;
     if (!kwave_shape(M, N, K) || !A || !B || !C || (((uintptr_t)A | (uintptr_t)B) & 15)) return SGPU_ERR_INVALID_ARG;
-    int rc;
-    if (pieces_taken(A, B, C, M, N, K, stream, &rc)) return rc;
     return kwave_launch(0, A, B, C, M, N, K, stream);
 }
 /* sgemm_kwave128's problems: M, N multiples of 128, K a multiple of 32, a 128-row A panel and a
@@ -745,8 +740,6 @@ int sgpu_sgemm_kwave128(const float *A, const float *B, float *C, int M, int N, 
     if (M < 0 || N < 0 || K < 0) return SGPU_ERR_INVALID_ARG;
     if (M == 0 || N == 0) return SGPU_OK;
     if (!kwave128_shape(M, N, K) || !A || !B || !C || (((uintptr_t)A | (uintptr_t)B) & 15)) return SGPU_ERR_INVALID_ARG;
-    int rc;
-    if (pieces_taken(A, B, C, M, N, K, stream, &rc)) return rc;
     return sgemm_common(K_SGEMM_KWAVE128, "sgemm_kwave128", A, B, C, M, N, K, stream);
 }
 /* The bf16-piece form (sgpu_pieces.hip): whole or shifted tiles of 128 rows and 128 or 256
@@ -805,14 +798,10 @@ static int pieces_win(const pieces_plan *p, int M, int N, int K, int cus) {
     const double member = byround > 1.35 * flat ? 1.35 * flat : byround > flat ? byround : flat;
     return p->us + 1.0 < member;
 }
-/* For the launchers of large products (sgemm_opt256, sgemm_kwave, sgemm_kwave_edge, sgemm_kwave128
- * and what sgpu_sgemm_opt plans as one of these): 1 when the product was launched in its piece
- * form (*rc: the launch's status).  Without a workspace
- * the tail is not split, which can turn the choice. */
-static int pieces_taken(const float *A, const float *B, float *C, int M, int N, int K, void *stream, int *rc) {
-    if (!pieces_shape(M, N, K) || !A || !B || !C || (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 3)) return 0;
-    devstate *d = cur(rc);
-    if (!d) return 1;
+/* 1 when the product was launched in its piece form (*rc: the launch's status).  Without a
+ * workspace the tail is not split, which can turn the choice. */
+static int pieces_taken(devstate *d, const float *A, const float *B, float *C, int M, int N, int K, void *stream, int *rc) {
+    if (!pieces_shape(M, N, K) || (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 3)) return 0;
     pieces_plan p = pieces_best(M, N, K, d->cus, 1);
     float *ws = NULL;
     unsigned *cnt = NULL;
@@ -847,8 +836,6 @@ int sgpu_sgemm_kwave_edge(const float *A, const float *B, float *C, int M, int N
     if (M == 0 || N == 0) return SGPU_OK;
     if (!kwave_edge_shape(M, N, K) || !A || !B || !C || (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 3))
         return SGPU_ERR_INVALID_ARG;
-    int rc;
-    if (pieces_taken(A, B, C, M, N, K, stream, &rc)) return rc;
     return kwave_launch(1, A, B, C, M, N, K, stream);
 }
 /* The optimised entry picks the member with the least work on its busiest CU: tiles are one
@@ -1086,7 +1073,8 @@ const char *sgpu_sgemm_opt_plan(int M, int N, int K, int cus, int *splits) {
     return g_sgemm_members[p].name;
 }
 
-/* The plans whose product may run in its piece form. */
+/* The plans whose product may run in its piece form (the members' own launchers never do: they use no
+ * workspace and allocate nothing). */
 static int plan_large(int p) {
     if (p >= 0) return g_sgemm_members[p].kid == K_SGEMM_OPT || g_sgemm_members[p].kid == K_SGEMM_OPT256;
     return p == PLAN_KWAVE128 || p == PLAN_KWAVE || p == PLAN_KWAVE_EDGE;
@@ -1113,7 +1101,7 @@ int sgpu_sgemm_opt(const float *A, const float *B, float *C, int M, int N, int K
     unsigned *cnt;
     if (p == PLAN_SPLITK && sk_workspace(d, stream, &ws, &cnt) == SGPU_OK)    /* else: the unsplit member */
         return splitk_launch(d, A, B, C, M, N, K, S, ws, cnt, stream);
-    if (plan_large(p) && pieces_taken(A, B, C, M, N, K, stream, &rc)) return rc;
+    if (plan_large(p) && pieces_taken(d, A, B, C, M, N, K, stream, &rc)) return rc;
     if (p == PLAN_KWAVE128 && !(((uintptr_t)A | (uintptr_t)B) & 15))
         return sgemm_common(K_SGEMM_KWAVE128, "sgemm_kwave128", A, B, C, M, N, K, stream);
     if (p == PLAN_KWAVE && !(((uintptr_t)A | (uintptr_t)B) & 15)) return kwave_launch(0, A, B, C, M, N, K, stream);

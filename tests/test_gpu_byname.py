@@ -271,6 +271,28 @@ def test_kwave_members_by_name_any_grid(gpu, hip, sym, M, N, K, grid):
     assert np.array_equal(dC.to_host(), want)
 
 
+@pytest.mark.parametrize("sym,M,N,K", [("sgemm_kwave128", 2048, 2048, 2048), ("sgemm_kwave", 3072, 3072, 1024),
+                                       ("sgemm_kwave_edge", 2047, 2049, 2048), ("sgemm_opt256", 4096, 4096, 1024)])
+def test_member_launchers_launch_their_own_kernel(gpu, hip, sym, M, N, K):
+    """The members' own launchers run the fp32 kernel of their name (no workspace, no other member)
+    also where sgpu_sgemm_opt would take the piece form: on random floats C equals, bit for bit, the
+    symbol launched from its code object at its published geometry."""
+    say(f"launcher against symbol {sym} {M}x{N}x{K}")
+    assert gpu.lib().sgpu_sgemm_opt_pieces(M, N, K, gpu.device_props().compute_units)
+    rng = np.random.default_rng(M + N + K)
+    dA = upload(gpu, rng.uniform(-1, 1, (M, K)).astype(np.float32))
+    dB = upload(gpu, rng.uniform(-1, 1, (K, N)).astype(np.float32))
+    dC, dD = gpu.DeviceArray((M, N)), gpu.DeviceArray((M, N))
+    dC.fill_bytes(0xFF)
+    gpu.call("sgpu_" + sym, dA.ptr, dB.ptr, dC.ptr, M, N, K, None)
+    grid, block = (ct.c_uint * 3)(), (ct.c_uint * 3)()
+    gpu.call("sgpu_kernel_geometry", sym.encode(), M, N, K, grid, block)
+    assert list(block) == [256, 1, 1]
+    hip.launch(hip.function("switch_gpu", sym), (grid[0], grid[1]), [Ptr(dA.ptr), Ptr(dB.ptr), Ptr(dD.ptr), M, N, K])
+    gpu.synchronize()
+    assert np.array_equal(dC.to_host(), dD.to_host())
+
+
 def test_block_beyond_launch_bound_refused(gpu, hip):
     """The kernels' block-size checks (sgpu_block256) read no z size: a block of x*y == 256
     threads has z == 1 because HIP refuses a launch whose block holds more threads than the

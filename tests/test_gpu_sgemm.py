@@ -128,8 +128,8 @@ def test_tile_paths_integer_exact(gpu, fn, M, N, K):
     assert np.array_equal(C, (A.astype(np.float64) @ B.astype(np.float64)).astype(np.float32))
 
 
-# sgpu_sgemm_opt launches what sgpu_sgemm_opt_plan names for this device: on float inputs its
-# C equals the named launch's bit for bit.  A split sums its partials in split order, so a
+# sgpu_sgemm_opt launches what sgpu_sgemm_opt_plan names for this device, or the piece form where
+# sgpu_sgemm_opt_pieces names it: on float inputs its C equals the named launch's bit for bit.  A split sums its partials in split order, so a
 # split C differs from the unsplit member's, and a different split count would differ too.
 PLAN_SHAPES = [(1023, 1025, 997), (768, 768, 2048), (1000, 1000, 1000), (1088, 1024, 1024), (1024, 1024, 1000),
                (8192, 128, 1000), (1023, 1025, 128),
@@ -155,6 +155,8 @@ def test_opt_launches_its_plan(gpu, M, N, K):
         gpu.call("sgpu_sgemm_splitk", dA.ptr, dB.ptr, dD.ptr, M, N, K, S.value, None)
     elif name in ("sgemm_small16", "sgemm_small32"):
         gpu.call("sgpu_sgemm_small", dA.ptr, dB.ptr, dD.ptr, M, N, K, int(name[-2:]), None)
+    elif gpu.lib().sgpu_sgemm_opt_pieces(M, N, K, cus):
+        gpu.call("sgpu_sgemm_pieces", dA.ptr, dB.ptr, dD.ptr, M, N, K, None)
     else:
         gpu.call("sgpu_" + name, dA.ptr, dB.ptr, dD.ptr, M, N, K, None)
     gpu.synchronize()
