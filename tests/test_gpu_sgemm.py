@@ -837,6 +837,24 @@ def test_pieces_integer_exact(gpu, M, N, K, a_off, b_off):
         assert np.array_equal(run_sgemm(gpu, "sgpu_sgemm_pieces", A, B, M, N, K, a_off, b_off), want)
 
 
+def test_pieces_products_of_single_terms(gpu):
+    """C = diag(d) B and products of constant matrices, whose left-out piece products no other term
+    averages away: at most 2^-24 of the product is left out, and the result is rounded once (and, 32
+    equal terms summed, a few times more: 4 x 2^-24 allowed for the sum)."""
+    n = 300
+    rng = np.random.default_rng(5)
+    d, B = rng.uniform(1, 2, n).astype(np.float32), rng.uniform(1, 2, (n, n)).astype(np.float32)
+    want = d[:, None].astype(np.float64) * B
+    got = run_sgemm(gpu, "sgpu_sgemm_pieces", np.diag(d), B, n, n, n)
+    assert (np.abs(got - want) / want).max() <= 2.02 * 2.0**-24      # + the small products' own sums
+    assert np.array_equal(run_sgemm(gpu, "sgpu_sgemm_pieces", np.eye(n, dtype=np.float32), B, n, n, n), B)
+    for x in (1 + 2.0**-8 - 2.0**-23, 1 + 2.0**-8 + 2.0**-16, 1.9999999):
+        A = np.full((128, 32), x, np.float32)
+        got = run_sgemm(gpu, "sgpu_sgemm_pieces", A, A.T.copy(), 128, 128, 32)
+        want = 32 * float(A[0, 0]) ** 2
+        assert (np.abs(got - want) / want).max() <= 6 * 2.0**-24
+
+
 @pytest.mark.parametrize("M,N,K", [(1024, 4097, 2048), (2049, 4111, 2000), (3073, 3073, 3073), (4097, 4097, 4097),
                                    (1090, 5147, 1751)])
 def test_pieces_overlap_has_one_owner(gpu, M, N, K):
