@@ -14,7 +14,9 @@
 // 2^-32 would cost 24% at 4096^3 (748 us against 602) and leave that error as it is.
 //
 // The cut needs normal-sized numbers.  Where it would lose bits that fp32 keeps, or meets what it
-// cannot represent, the elements concerned are computed again by serial fp32 FMAs:
+// cannot represent, the tile concerned is computed again on the fp32 matrix cores (a product whose
+// tiles all are: 2048^3 115 -> 290-310 us, fp32 members 152; 4096^3 0.69 -> 1.9-2.1 ms, members 1.1.  By
+// a serial dot product per element 2048^3 took 12.2 ms):
 //  * sums that come out non-finite (an infinity, a NaN, an operand that rounds up to infinity);
 //  * rows of A or columns of B whose largest magnitude is below 2^-100 (bf16 subnormals end at
 //    2^-133), and row-column pairs whose largest product is below 2^-96.
@@ -48,10 +50,65 @@ __device__ __forceinline__ void cut2(float x0, float x1, uint32_t (&p)[3]) {
 }
 __device__ __forceinline__ float max3abs(float m, float a, float b) { return fmaxf(fmaxf(m, fabsf(a)), fabsf(b)); }
 
-__device__ __noinline__ float serial_dot(const float* __restrict__ a, const float* __restrict__ b, int K, int N) {
-    float acc = 0.0f;
-    for (int k = 0; k < K; k++) acc = __builtin_fmaf(a[k], b[(size_t)k * N], acc);
-    return acc;
+// The wave's part of a tile again on the fp32 matrix cores, from memory: a points at the lane's first
+// row of A (its others 16 rows on), b at its first column of B.  Lane quarter q takes k 4 q.. of each
+// 16 (the k order within an MFMA is free), so operands are whole vectors; the next 16 k are loaded under
+// this one's MFMAs.
+template <int NJ>
+__device__ __forceinline__ void fp32_tile(const float* __restrict__ a, const float* __restrict__ b, int K, int N, int quarter,
+                                          f32x4 (&acc)[4][NJ]) {
+    typedef float rowv __attribute__((ext_vector_type(NJ)));
+    typedef float rowv_a4 __attribute__((ext_vector_type(NJ), aligned(4)));
+    a += 4 * quarter;
+    b += (size_t)(4 * quarter) * N;
+    f32x4 av[2][4], sum[4][NJ];
+    rowv bv[2][4];
+    // slice s of 16 k; the last starts at K - 16 (K >= 32), its k already summed are set to zero
+    auto load = [&](int s, int u) __attribute__((always_inline)) {
+        const int k = min(16 * s, K - 16);
+#pragma unroll
+        for (int i = 0; i < 4; i++) av[u][i] = *reinterpret_cast<const sgpu_f32x4_a4*>(a + (size_t)(16 * i) * K + k);
+#pragma unroll
+        for (int t = 0; t < 4; t++) bv[u][t] = *reinterpret_cast<const rowv_a4*>(b + (size_t)(k + t) * N);
+    };
+    auto mul = [&](int s, int u) __attribute__((always_inline)) {
+        const int done = 16 * s - (K - 16);
+        if (done > 0) {
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+                if (4 * quarter + t < done) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) av[u][i][t] = 0.0f;
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) bv[u][t][j] = 0.0f;
+                }
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++)
+                    sum[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u][i][t], bv[u][t][j], sum[i][j], 0, 0, 0);
+    };
+    const int ns = (K + 15) / 16;
+    load(0, 0);
+    for (int s0 = 0; s0 < ns; s0 += 16) {                  // sums of 256 k, added up
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) sum[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int s = s0; s < min(s0 + 16, ns); s += 2) {
+            load(s + 1, 1);
+            mul(s, 0);
+            load(s + 2, 0);
+            mul(s + 1, 1);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) acc[i][j] = s0 == 0 ? sum[i][j] : acc[i][j] + sum[i][j];
+    }
 }
 
 // Bound: the matrix cores.  A block of 2x4 waves computes a tile of 128 x 64 NJ, a wave 64 x 16 NJ of
@@ -203,6 +260,8 @@ __device__ __forceinline__ void sgemm_pieces(const float* __restrict__ A, const 
 
     // The largest magnitude of each of the tile's rows and columns, through LDS.
     float* const rmax = reinterpret_cast<float*>(as[0]);   // 128 rows, then TN columns
+    float& redo = rmax[TM + TN];                           // 1: the tile is computed again
+    if (tid == 0) redo = 0.0f;
 #pragma unroll
     for (int i = 0; i < 2; i++) {
 #pragma unroll
@@ -280,24 +339,30 @@ __device__ __forceinline__ void sgemm_pieces(const float* __restrict__ A, const 
     float cmax[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; j++) cmax[j] = rmax[TM + lc + j];
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float ra = rmax[64 * wm + 16 * i + 4 * quarter + e];
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+                bad |= !__builtin_isfinite(acc[i][j][e]) ||
+                       (fminf(fminf(ra, cmax[j]) * 0x1p100f, ra * cmax[j] * 0x1p96f) < 1.0f && ra > 0.0f && cmax[j] > 0.0f);
+        }
+    if (__any(bad) && lane == 0) redo = 1.0f;
+    __syncthreads();
+    if (redo != 0.0f) fp32_tile<NJ>(A + (size_t)(m0 + 64 * wm + l16) * K, B + n, K, N, quarter, acc);
     auto store = [&](auto shifted) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const int lm = 64 * wm + 16 * i + 4 * quarter + e, m = m0 + lm;
-                const float ra = rmax[lm];
+                const int m = m0 + 64 * wm + 16 * i + 4 * quarter + e;
                 if (shifted && m < mt) continue;
                 rowv v;
-                bool redo = false;
 #pragma unroll
-                for (int j = 0; j < NJ; j++) {
-                    v[j] = acc[i][j][e];
-                    redo |= !__builtin_isfinite(v[j]) || (fminf(fminf(ra, cmax[j]) * 0x1p100f, ra * cmax[j] * 0x1p96f) < 1.0f &&
-                                                          ra > 0.0f && cmax[j] > 0.0f);
-                }
-                if (redo)
-                    for (int j = 0; j < NJ; j++) v[j] = serial_dot(A + (size_t)m * K, B + n + j, K, N);
+                for (int j = 0; j < NJ; j++) v[j] = acc[i][j][e];
                 float* const c = C + (size_t)m * N + n;
                 if (!shifted || n >= nt) {
                     *reinterpret_cast<rowv_a4*>(c) = v;

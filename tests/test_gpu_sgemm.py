@@ -914,7 +914,28 @@ def test_pieces_scales(gpu, scale_a, scale_b):
     assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want) + 64 * 2.0**-149 * np.sqrt(M * N)
 
 
-@pytest.mark.parametrize("M,N,K", [(128, 128, 64), (300, 257, 100), (2047, 2049, 130)])
+def test_pieces_odd_inputs_cost_a_second_product_at_most(gpu):
+    """A product whose every tile has to be computed again takes a few times the plain one's time
+    (about 3, on the fp32 matrix cores; element by element it took a hundred times)."""
+    n = 2048
+    rng = np.random.default_rng(1)
+    A, B = rng.uniform(-1, 1, (n, n)).astype(np.float32), rng.uniform(-1, 1, (n, n)).astype(np.float32)
+    dB, dC, ev, ms = gpu.DeviceArray.from_host(B), gpu.DeviceArray((n, n)), gpu.Events(), []
+    for a in (A, np.full_like(A, np.nan)):
+        dA = gpu.DeviceArray.from_host(a)
+        gpu.call("sgpu_sgemm_pieces", dA.ptr, dB.ptr, dC.ptr, n, n, n, None)
+        ev.record_start()
+        for _ in range(5):
+            gpu.call("sgpu_sgemm_pieces", dA.ptr, dB.ptr, dC.ptr, n, n, n, None)
+        ev.record_stop()
+        gpu.synchronize()
+        ms.append(ev.elapsed_ms())
+    say("plain, all NaN (ms):", ms)
+    assert np.isnan(dC.to_host()).all() and ms[1] < 10 * ms[0]
+
+
+@pytest.mark.parametrize("M,N,K", [(128, 128, 64), (300, 257, 100), (2047, 2049, 130), (129, 300, 33), (255, 513, 993),
+                                   (2047, 2049, 300)])
 def test_pieces_nonfinite_and_nan_padding(gpu, M, N, K):
     """Non-finite operands as IEEE fp32 has them, a row of A of zeros, and operands that are
     followed by NaN: no load passes their ends."""
