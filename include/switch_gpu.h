@@ -191,10 +191,13 @@ int sgpu_sgemm_kwave_edge(const float *A, const float *B, float *C, int M, int N
  * counterpart in the reference: an added member of the family with the (A, B, C, M, N, K)
  * symbol arguments. */
 int sgpu_sgemm_kwave128(const float *A, const float *B, float *C, int M, int N, int K, void *stream);
-/* The same product on the bf16 matrix cores: every operand cut without loss into three bf16
- * pieces, six exact piece products summed in fp32, 128x128 tiles (results as close to the exact
- * product as the fp32 members'; non-finite sums, and rows or columns of numbers too small to
- * cut, by serial fp32 FMAs).  M, N >= 128, K >= 32, float-aligned A, B, C
+/* The same product on the bf16 matrix cores: every operand cut into three bf16 pieces (all of its
+ * 24 bits from 2^-110 up), six piece products summed in fp32, 128x128 tiles.  At most 2^-24 of a
+ * product is left out, so a sum of one term may be two roundings from the exact one where the fp32
+ * members' is one; sums of many terms end closer to the exact ones than theirs.  What bf16 cannot
+ * hold -- non-finite sums, elements that numbers below 2^-110 or products below 2^-110 could
+ * matter to -- is computed again on the fp32 matrix cores (two to three times as long where a
+ * whole product is).  M, N >= 128, K >= 32, float-aligned A, B, C
  * (SGPU_ERR_INVALID_ARG otherwise; M or N == 0 is a no-op).  The tiles past the last full round
  * of compute units are split over K through the stream's split-K workspace; a stream that has
  * none and cannot get one runs them unsplit.  No counterpart in the reference. */

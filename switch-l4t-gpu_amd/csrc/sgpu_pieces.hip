@@ -13,13 +13,17 @@
 // (4096^3 3.8e-7 against 5.7e-7), those of a single term up to 2 x 2^-24 away.  All eight that reach
 // 2^-32 would cost 24% at 4096^3 (748 us against 602) and leave that error as it is.
 //
-// The cut needs normal-sized numbers.  Where it would lose bits that fp32 keeps, or meets what it
-// cannot represent, the tile concerned is computed again on the fp32 matrix cores (a product whose
-// tiles all are: 2048^3 115 -> 290-310 us, fp32 members 152; 4096^3 0.69 -> 1.9-2.1 ms, members 1.1.  By
-// a serial dot product per element 2048^3 took 12.2 ms):
-//  * sums that come out non-finite (an infinity, a NaN, an operand that rounds up to infinity);
-//  * rows of A or columns of B whose largest magnitude is below 2^-100 (bf16 subnormals end at
-//    2^-133), and row-column pairs whose largest product is below 2^-96.
+// bf16 pieces end at 2^-133 (their subnormals count), so numbers below 2^-110 may lose bits that fp32
+// keeps, and the largest round up to infinity.  A wave's part of a tile is computed again on the fp32
+// matrix cores where it holds
+//  * a sum that came out non-finite (an infinity, a NaN, an operand that rounded up to infinity);
+//  * an element whose row of A or column of B lost bits, if it is below K 2^-108 times the other
+//    operand's largest magnitude there: what was lost, 2^-133 a number, could pass 2^-25 of it;
+//  * an element whose row and column are nonzero with the product of their largest magnitudes below
+//    2^-110 (products of pieces end at 2^-149).
+// A product all of which is computed again: 2048^3 110 -> 285-308 us (fp32 members 151), 4096^3 0.67 ->
+// 1.9-2.1 ms (1.1); with one NaN in A 180 us and 1.13 ms.  By a serial dot product per element 2048^3
+// took 12.2 ms and 0.8.
 #include "sgpu_device.h"
 
 namespace {
@@ -38,8 +42,9 @@ struct bool_c {
 };
 
 // The three pieces of two numbers, packed: two rounded to nearest, then the upper halves of what is
-// left (8 bits at most), which one v_perm takes for two numbers.
-__device__ __forceinline__ void cut2(float x0, float x1, uint32_t (&p)[3]) {
+// left (8 bits at most), which one v_perm takes for two numbers.  What that drops (numbers below
+// 2^-110 only) is seen in the lower halves.
+__device__ __forceinline__ void cut2(float x0, float x1, uint32_t (&p)[3], uint32_t& lost) {
     p[0] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x0, x1}, bf16x2));
     x0 -= __uint_as_float(p[0] << 16);
     x1 -= __uint_as_float(p[0] & 0xffff0000u);
@@ -47,7 +52,9 @@ __device__ __forceinline__ void cut2(float x0, float x1, uint32_t (&p)[3]) {
     x0 -= __uint_as_float(p[1] << 16);
     x1 -= __uint_as_float(p[1] & 0xffff0000u);
     p[2] = __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u);
+    lost |= __float_as_uint(x0) | __float_as_uint(x1);
 }
+constexpr float kTiny = 0x1p-55f;                      // rows and columns from here on need no look at their products
 __device__ __forceinline__ float max3abs(float m, float a, float b) { return fmaxf(fmaxf(m, fabsf(a)), fabsf(b)); }
 
 // The wave's part of a tile again on the fp32 matrix cores, from memory: a points at the lane's first
@@ -140,6 +147,7 @@ __device__ __forceinline__ void sgemm_pieces(const float* __restrict__ A, const 
     typedef float rowv __attribute__((ext_vector_type(NJ)));
     typedef float rowv_a4 __attribute__((ext_vector_type(NJ), aligned(4)));
     __shared__ __attribute__((aligned(1024))) uint16_t as[2][3 * TM * KS], bs[2][3 * TN * KS];
+    __shared__ int look;                                   // some row or column lost bits or is tiny
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, quarter = lane >> 4, wm = wave >> 2, wn = wave & 3;
     // Blocks are dealt round-robin to the 8 XCDs: of the unsplit tiles each XCD takes a contiguous
@@ -180,22 +188,23 @@ __device__ __forceinline__ void sgemm_pieces(const float* __restrict__ A, const 
             for (int c = 0; c < NJ; c++) bv[e][c] = 0.0f;
         }
     };
+    uint32_t lost_a = 0, lost_b = 0;
     float amax[2] = {0.0f, 0.0f}, bmax[NJ];
 #pragma unroll
     for (int c = 0; c < NJ; c++) bmax[c] = 0.0f;
     const int wo = r * KS + 8 * ((q >> 1) ^ (-(r >> 2) & 3)) + 4 * (q & 1);
     auto cut_a = [&](int buf, int i) __attribute__((always_inline)) {
         uint32_t lo[3], hi[3];
-        cut2(av[i][0], av[i][1], lo);
-        cut2(av[i][2], av[i][3], hi);
+        cut2(av[i][0], av[i][1], lo, lost_a);
+        cut2(av[i][2], av[i][3], hi, lost_a);
 #pragma unroll
         for (int p = 0; p < 3; p++) *reinterpret_cast<u32x2*>(as[buf] + wo + (p * TM + 64 * i) * KS) = u32x2{lo[p], hi[p]};
         amax[i] = max3abs(max3abs(amax[i], av[i][0], av[i][1]), av[i][2], av[i][3]);
     };
     auto cut_b = [&](int buf, int c) __attribute__((always_inline)) {
         uint32_t lo[3], hi[3];
-        cut2(bv[0][c], bv[1][c], lo);
-        cut2(bv[2][c], bv[3][c], hi);
+        cut2(bv[0][c], bv[1][c], lo, lost_b);
+        cut2(bv[2][c], bv[3][c], hi, lost_b);
 #pragma unroll
         for (int p = 0; p < 3; p++) *reinterpret_cast<u32x2*>(bs[buf] + wo + (p * TN + 64 * c) * KS) = u32x2{lo[p], hi[p]};
         bmax[c] = max3abs(max3abs(bmax[c], bv[0][c], bv[1][c]), bv[2][c], bv[3][c]);
@@ -243,6 +252,7 @@ __device__ __forceinline__ void sgemm_pieces(const float* __restrict__ A, const 
         }
         __syncthreads();
     };
+    if (tid == 0) look = 0;
     load_a(s0);
     load_b(s0);
     mask(s0);
@@ -258,22 +268,25 @@ __device__ __forceinline__ void sgemm_pieces(const float* __restrict__ A, const 
         if (s + 1 < nk) step(s + 1, 1);
     }
 
-    // The largest magnitude of each of the tile's rows and columns, through LDS.
+    // The largest magnitude of each of the tile's rows and columns, through LDS; negative where bits
+    // were lost.
     float* const rmax = reinterpret_cast<float*>(as[0]);   // 128 rows, then TN columns
-    float& redo = rmax[TM + TN];                           // 1: the tile is computed again
-    if (tid == 0) redo = 0.0f;
+    auto put_max = [&](int at, float m, uint32_t lost) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
+        for (int o = 1; o < 8; o *= 2) m = fmaxf(m, __shfl_xor(m, o));
+        lost = (lost & 0xffffu) != 0u;
+        if (q == 0) rmax[at] = lost ? -m : m;
+        if (lost || (m < kTiny && m > 0.0f)) look = 1;
+    };
 #pragma unroll
-        for (int o = 1; o < 8; o *= 2) amax[i] = fmaxf(amax[i], __shfl_xor(amax[i], o));
-        if (q == 0) rmax[r + 64 * i] = amax[i];
+    for (int o = 1; o < 8; o *= 2) {
+        lost_a |= (uint32_t)__shfl_xor((int)lost_a, o);
+        lost_b |= (uint32_t)__shfl_xor((int)lost_b, o);
     }
 #pragma unroll
-    for (int c = 0; c < NJ; c++) {
+    for (int i = 0; i < 2; i++) put_max(r + 64 * i, amax[i], lost_a);
 #pragma unroll
-        for (int o = 1; o < 8; o *= 2) bmax[c] = fmaxf(bmax[c], __shfl_xor(bmax[c], o));
-        if (q == 0) rmax[TM + NJ * r + c] = bmax[c];
-    }
+    for (int c = 0; c < NJ; c++) put_max(TM + NJ * r + c, bmax[c], lost_b);
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -304,6 +317,7 @@ __device__ __forceinline__ void sgemm_pieces(const float* __restrict__ A, const 
         // issued before the first add
         constexpr int U = 4 / NJ;
         float big = 0.0f;
+        bool lost = false;
         for (int s2 = 0; s2 < S; s2 += U) {
             f32x4 v[U][4][NJ];
             float m[U];
@@ -323,36 +337,47 @@ __device__ __forceinline__ void sgemm_pieces(const float* __restrict__ A, const 
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 if (s2 + u >= S) break;
-                big = fmaxf(big, m[u]);
+                big = fmaxf(big, fabsf(m[u]));
+                lost |= m[u] < 0.0f;
 #pragma unroll
                 for (int i = 0; i < 4; i++)
 #pragma unroll
                     for (int j = 0; j < NJ; j++) acc[i][j] = s2 + u == 0 ? v[u][i][j] : acc[i][j] + v[u][i][j];
             }
         }
-        if (tid < TM + TN) rmax[tid] = big;
+        if (tid < TM + TN) rmax[tid] = lost ? -big : big;
+        if (lost || (big < kTiny && big > 0.0f)) look = 1;
         if (tid == 0) __hip_atomic_store(cnt + part, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
     }
     // Accumulator e of tile (i, j): row 64 wm + 16 i + 4 quarter + e, column NJ (16 wn + l16) + j.
     const int lc = NJ * (16 * wn + l16), n = n0 + lc;
-    float cmax[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; j++) cmax[j] = rmax[TM + lc + j];
-    bool bad = false;
+    uint32_t top = 0;
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const float ra = rmax[64 * wm + 16 * i + 4 * quarter + e];
+        for (int j = 0; j < NJ; j++)
 #pragma unroll
-            for (int j = 0; j < NJ; j++)
-                bad |= !__builtin_isfinite(acc[i][j][e]) ||
-                       (fminf(fminf(ra, cmax[j]) * 0x1p100f, ra * cmax[j] * 0x1p96f) < 1.0f && ra > 0.0f && cmax[j] > 0.0f);
+            for (int e = 0; e < 4; e++) top = max(top, __float_as_uint(acc[i][j][e]) & 0x7fffffffu);
+    bool again = top >= 0x7f800000u;
+    if (look) {
+        const float least = (float)K * 0x1p-108f;
+        for (int j = 0; j < NJ; j++) {
+            const float cm = rmax[TM + lc + j], ca = fabsf(cm);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float rm = rmax[64 * wm + 16 * i + 4 * quarter + e], ra = fabsf(rm);
+                    float v = 0.0f;
+#pragma unroll
+                    for (int jj = 0; jj < NJ; jj++) v = jj == j ? fabsf(acc[i][jj][e]) : v;
+                    again |= (rm < 0.0f && v < least * ca) || (cm < 0.0f && v < least * ra) ||
+                             (ra > 0.0f && ca > 0.0f && ra * ca < 0x1p-110f);
+                }
         }
-    if (__any(bad) && lane == 0) redo = 1.0f;
-    __syncthreads();
-    if (redo != 0.0f) fp32_tile<NJ>(A + (size_t)(m0 + 64 * wm + l16) * K, B + n, K, N, quarter, acc);
+    }
+    if (__any(again)) fp32_tile<NJ>(A + (size_t)(m0 + 64 * wm + l16) * K, B + n, K, N, quarter, acc);
     auto store = [&](auto shifted) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 4; i++)

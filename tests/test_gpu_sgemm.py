@@ -914,6 +914,28 @@ def test_pieces_scales(gpu, scale_a, scale_b):
     assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want) + 64 * 2.0**-149 * np.sqrt(M * N)
 
 
+@pytest.mark.parametrize("n,K", [(300, 300), (128, 500)])
+def test_pieces_small_numbers_beside_large_ones(gpu, n, K):
+    """Numbers below 2^-110, which three bf16 pieces do not hold, in rows and columns that hold ones
+    as well: identity times B and A times identity give them back as they are (subnormal ones too),
+    and 2^-135 * 2^120 counts where nothing larger does."""
+    rng = np.random.default_rng(n)
+    X = rng.choice([-1, 1], (n, n)) * rng.uniform(1, 2, (n, n)) * 2.0 ** rng.choice([0, -100, -111, -120, -126, -135, -140], (n, n))
+    X = X.astype(np.float32)
+    eye = np.zeros((n, K), np.float32)
+    at = np.arange(n) * (K // n)
+    eye[np.arange(n), at] = 1
+    B = np.zeros((K, n), np.float32)
+    B[at] = X
+    assert np.array_equal(run_sgemm(gpu, "sgpu_sgemm_pieces", eye, B, n, n, K), X)
+    assert np.array_equal(run_sgemm(gpu, "sgpu_sgemm_pieces", B.T.copy(), eye.T.copy(), n, n, K), X.T)
+    A, B = np.zeros((n, K), np.float32), np.zeros((K, n), np.float32)
+    A[:, 0], A[:, 1], B[0, ::2], B[1] = 1, 2.0**-135, 1, 2.0**120
+    want = np.tile(np.where(np.arange(n) % 2, 2.0**-15, 1 + 2.0**-15), (n, 1)).astype(np.float32)
+    assert np.array_equal(run_sgemm(gpu, "sgpu_sgemm_pieces", A, B, n, n, K), want)
+    assert np.array_equal(run_sgemm(gpu, "sgpu_sgemm_pieces", B.T.copy(), A.T.copy(), n, n, K), want.T)
+
+
 def test_pieces_odd_inputs_cost_a_second_product_at_most(gpu):
     """A product whose every tile has to be computed again takes a few times the plain one's time
     (about 3, on the fp32 matrix cores; element by element it took a hundred times)."""
