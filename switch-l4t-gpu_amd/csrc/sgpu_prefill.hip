@@ -371,7 +371,8 @@ __device__ __forceinline__ void pf_mm(const uint16_t* __restrict__ W, const uint
 //    consecutive dims per lane: one 4*NB-byte load per step).
 // K and V of the wave's next tile are loaded while this tile's softmax and second product run.
 // Loads go through buffer resources that end at the last valid key row: rows past it read as
-// zero and are masked.  The heavy blocks (last rows) are dispatched first.
+// zero and are masked.  In tiles that reach past some row's own position, non-finite values of V are
+// taken out of the product (0 times an infinity is a NaN) and added at the end to the rows that see them.  The heavy blocks (last rows) are dispatched first.
 // Measured against one block per head and row on the vector ALUs, which read K and V once per
 // row, 14 query and 2 KV heads of 64: 50 -> 16 us a launch at 500 rows, 1390 -> 172 us for 3001 rows
 // (194 with expf and with a lane's dims of K in one run).
@@ -384,6 +385,7 @@ __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const flo
     typedef uint32_t vseg __attribute__((ext_vector_type(NB)));
     __shared__ float part[4][32][PITCH];
     __shared__ float ml[4][2][32];
+    __shared__ int odd[4];                            // per wave: some V was taken out
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l32 = lane & 31, h = lane >> 5;
     const int head = blockIdx.x % NH, q0 = ((T + 31) / 32 - 1 - blockIdx.x / NH) * 32;
@@ -434,6 +436,7 @@ __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const flo
 #pragma unroll
         for (int r = 0; r < 16; r++) o[j][r] = 0.0f;
     float m = -INFINITY, l = 0.0f;
+    bool taken = false;                               // non-finite V taken out of a tile
     load_k(wave);
     load_v(wave);
     for (int t = wave; t < ntile; t += 4) {
@@ -449,7 +452,8 @@ __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const flo
         float mx = -INFINITY;
 #pragma unroll
         for (int r = 0; r < 16; r++) s[r] = (s[r] + s1[r]) * scale2;
-        if (32 * t + 31 > pos0 + q0) {                // the tile reaches past some row's own position
+        const bool past = 32 * t + 31 > pos0 + q0;    // the tile reaches past some row's own position
+        if (past) {
 #pragma unroll
             for (int r = 0; r < 16; r++)
                 if (32 * t + 8 * (r / 4) + 4 * h + r % 4 > qpos) s[r] = -INFINITY;
@@ -473,6 +477,16 @@ __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const flo
 #pragma unroll
                 for (int r = 0; r < 16; r++) o[j][r] *= al;
         }
+        if (past) {                                   // a weight of zero must not meet an infinity or a NaN
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+#pragma unroll
+                for (int j = 0; j < NB; j++) {
+                    const bool odd = (vr[r][j] & 0x7f800000u) == 0x7f800000u;
+                    taken |= odd;
+                    vr[r][j] = odd ? 0u : vr[r][j];
+                }
+        }
 #pragma unroll
         for (int r = 0; r < 16; r++)
 #pragma unroll
@@ -481,6 +495,8 @@ __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const flo
         load_v(t + 4);
     }
     l += __shfl_xor(l, 32);
+    taken = __any(taken);
+    if (lane == 0) odd[wave] = taken;
     if (h == 0) {
         ml[wave][0][l32] = m;
         ml[wave][1][l32] = l;
@@ -514,6 +530,25 @@ __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const flo
         mag = max(mag, mag_bits(v[e]));
     }
     const size_t C = (size_t)NH * HD, t = q0 + q, c = (size_t)head * HD + d0;
+    if (odd[0] | odd[1] | odd[2] | odd[3]) {          // the V taken out, to the rows that see them
+        for (int k = (pos0 + q0 + 1) / 32 * 32; k <= pos0 + (int)t; k++) {
+            const size_t kv = (size_t)k * KVD + (size_t)g * HD;
+            bool any = false;
+            for (int e = 0; e < HD / 8; e++) any |= !__builtin_isfinite(vc[kv + d0 + e]);
+            if (!any) continue;
+            float s = 0.0f;
+            for (int d = 0; d < HD; d++) s = __builtin_fmaf(qkv[t * QKVD + (size_t)head * HD + d], kc[kv + d], s);
+            const float w = __builtin_amdgcn_exp2f(s * scale2 - M) / L;
+#pragma unroll
+            for (int e = 0; e < HD / 8; e++) {
+                const float x = vc[kv + d0 + e];
+                v[e] = __builtin_isfinite(x) ? v[e] : __builtin_fmaf(w, x, v[e]);
+            }
+        }
+        mag = 0;
+#pragma unroll
+        for (int e = 0; e < HD / 8; e++) mag = max(mag, mag_bits(v[e]));
+    }
     if constexpr (HD >= G) {
         if (P) {                                      // block-uniform; a 64-block is 8 or 4 threads of one row
 #pragma unroll

@@ -202,6 +202,29 @@ def test_engine_batched_prefill(gpu, og):
     eng.close()
 
 
+@pytest.mark.parametrize("T,bad,value", [(40, 20, np.nan), (64, 33, np.inf), (64, 63, -np.inf), (31, 1, np.nan)])
+def test_engine_prefill_nonfinite_row_stays_causal(gpu, og, T, bad, value):
+    """A prompt row whose embedding is not finite (so its k and v are not) leaves the rows before
+    it as they were: decoding on from that position with another token matches the CPU golden that
+    never saw the bad row."""
+    cfg = SMALL
+    w = unit_gain_weights(gpu, cfg, 31)
+    rng = np.random.default_rng(T)
+    ids = [int(v) for v in rng.integers(0, cfg["V"] - 1, T)]
+    ids[bad] = cfg["V"] - 1
+    w[(cfg["V"] - 1) * cfg["C"] + 5] = value
+    say("non-finite prompt row", bad, "of", T)
+    eng = gpu.Gpt2Engine(gpu.gpt2_cfg(**cfg), w)
+    gold = og.Gpt2Golden(og.gpt2_cfg(**cfg), w, NT)
+    assert not np.isfinite(eng.prefill(ids)).any()
+    for p in range(bad):
+        gold.forward(ids[p], p, False)
+    # the tied head's last row is not finite: its logit is left out
+    got, want = eng.forward(7, bad)[:-1], gold.forward(7, bad, True)[:-1]
+    assert np.isfinite(want).all() and np.abs(got - want).max() <= 1e-4 * np.abs(want).max()
+    eng.close()
+
+
 def test_engine_full_greedy_token_identical(gpu, og):
     cfg = gpu.gpt2_cfg()
     say("building GPT-2 124M random weights")
