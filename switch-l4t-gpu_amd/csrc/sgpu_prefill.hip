@@ -373,6 +373,11 @@ __device__ __forceinline__ void pf_mm(const uint16_t* __restrict__ W, const uint
 // Loads go through buffer resources that end at the last valid key row: rows past it read as
 // zero and are masked.  In tiles that reach past some row's own position, non-finite values of V are
 // taken out of the product (0 times an infinity is a NaN) and added at the end to the rows that see them.  The heavy blocks (last rows) are dispatched first.
+// Sums are kept short, as the vector-ALU form's were: four accumulators for a score's dims, and a
+// tile's output summed by itself before it is added (logits against 64 bits, GPT-2, mean of 16 seeds:
+// 300 rows 5.64e-7 -> 5.59e-7, 1000 rows 6.25e-7 -> 6.17e-7, vector ALUs 5.61e-7 and 6.13e-7; Qwen, 3001
+// rows 7.9e-7 -> 7.0e-7; the time stays, 11.18 -> 11.10 ms, as long as the wave keeps to half a
+// SIMD's registers: 308 of them took 11.99).
 // Measured against one block per head and row on the vector ALUs, which read K and V once per
 // row, 14 query and 2 KV heads of 64: 50 -> 16 us a launch at 500 rows, 1390 -> 172 us for 3001 rows
 // (194 with expf and with a lane's dims of K in one run).
@@ -428,7 +433,9 @@ __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const flo
         }
     };
 
-    // The softmax in powers of two: scores carry log2(e), so a weight is one v_exp_f32.
+    // The softmax in powers of two: a weight is one FMA and one v_exp_f32, exp2(score * scale2 - max).  The
+    // product is not rounded before the subtraction, so weights near the maximum, which carry the sum,
+    // are exact to v_exp_f32's own rounding however large the scores are.
     const float scale2 = scale * 1.44269504088896340736f;
     f32x16 o[NB];
 #pragma unroll
@@ -440,18 +447,16 @@ __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const flo
     load_k(wave);
     load_v(wave);
     for (int t = wave; t < ntile; t += 4) {
-        f32x16 s, s1;
+        f32x16 s4[4], s;
 #pragma unroll
-        for (int r = 0; r < 16; r++) s[r] = s1[r] = 0.0f;
+        for (int r = 0; r < 16; r++) s4[0][r] = s4[1][r] = s4[2][r] = s4[3][r] = 0.0f;
 #pragma unroll
-        for (int k = 0; k < HH; k += 2) {             // two accumulators: no MFMA waits for the one before it
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[k / 4][k % 4], qv[k], s, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[k / 4][k % 4 + 1], qv[k + 1], s1, 0, 0, 0);
-        }
+        for (int k = 0; k < HH; k++)                  // four accumulators: no MFMA waits for the one before it
+            s4[k % 4] = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[k / 4][k % 4], qv[k], s4[k % 4], 0, 0, 0);
         load_k(t + 4);
         float mx = -INFINITY;
 #pragma unroll
-        for (int r = 0; r < 16; r++) s[r] = (s[r] + s1[r]) * scale2;
+        for (int r = 0; r < 16; r++) s[r] = (s4[0][r] + s4[1][r]) + (s4[2][r] + s4[3][r]);
         const bool past = 32 * t + 31 > pos0 + q0;    // the tile reaches past some row's own position
         if (past) {
 #pragma unroll
@@ -460,23 +465,17 @@ __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const flo
         }
 #pragma unroll
         for (int r = 0; r < 16; r++) mx = fmaxf(mx, s[r]);
-        mx = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32)));
+        mx = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32)) * scale2);
         const float base = mx == -INFINITY ? 0.0f : mx;   // every key so far masked: weights are all zero
         const float al = __builtin_amdgcn_exp2f(m - base);
         m = mx;
         float sum = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-            s[r] = __builtin_amdgcn_exp2f(s[r] - base);
+            s[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], scale2, -base));
             sum += s[r];
         }
         l = l * al + sum;
-        if (__any(al != 1.0f)) {
-#pragma unroll
-            for (int j = 0; j < NB; j++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) o[j][r] *= al;
-        }
         if (past) {                                   // a weight of zero must not meet an infinity or a NaN
 #pragma unroll
             for (int r = 0; r < 16; r++)
@@ -487,12 +486,22 @@ __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const flo
                     vr[r][j] = odd ? 0u : vr[r][j];
                 }
         }
+        // the tile's sum by itself, then added: chains of 32 keys instead of all of the wave's
+        f32x16 c[NB];
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) c[j][r] = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; r++)
 #pragma unroll
             for (int j = 0; j < NB; j++)
-                o[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(vr[r][j]), s[r], o[j], 0, 0, 0);
+                c[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(vr[r][j]), s[r], c[j], 0, 0, 0);
         load_v(t + 4);
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) o[j][r] = __builtin_fmaf(o[j][r], al, c[j][r]);
     }
     l += __shfl_xor(l, 32);
     taken = __any(taken);
@@ -538,7 +547,7 @@ __device__ __forceinline__ void pf_attn(const float* __restrict__ qkv, const flo
             if (!any) continue;
             float s = 0.0f;
             for (int d = 0; d < HD; d++) s = __builtin_fmaf(qkv[t * QKVD + (size_t)head * HD + d], kc[kv + d], s);
-            const float w = __builtin_amdgcn_exp2f(s * scale2 - M) / L;
+            const float w = __builtin_amdgcn_exp2f(__builtin_fmaf(s, scale2, -M)) / L;
 #pragma unroll
             for (int e = 0; e < HD / 8; e++) {
                 const float x = vc[kv + d0 + e];
@@ -653,7 +662,7 @@ __global__ void __launch_bounds__(256) sgpu_pf_rms(const float* __restrict__ x, 
 }  // extern "C"
 
 #define SGPU_PF_ATTN(HD)                                                                                              \
-    extern "C" __global__ void __launch_bounds__(256) sgpu_pf_attn##HD(                                               \
+    extern "C" __global__ void __launch_bounds__(256, (HD) <= 64 ? 2 : 1) sgpu_pf_attn##HD(                                               \
         const float* __restrict__ qkv, const float* __restrict__ kc, const float* __restrict__ vc,                    \
         float* __restrict__ out, uint16_t* __restrict__ P, float* __restrict__ pd, int pos0, int T, int NH, int NKV,   \
         float scale, int QKVD) {                                                                                      \

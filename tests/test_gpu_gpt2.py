@@ -225,6 +225,41 @@ def test_engine_prefill_nonfinite_row_stays_causal(gpu, og, T, bad, value):
     eng.close()
 
 
+@pytest.mark.parametrize("T", [7, 48])
+def test_engine_prefill_attention_of_large_scores(gpu, T):
+    """Scores of 1024 that differ by a few units, all exact in fp32 (+-1 embeddings, LayerNorm without
+    epsilon, selections for q, k and v): the attention weights depend on the differences alone, so
+    the logits are within 2e-6 of float64 (weights and their sum rounded a few times).  A score
+    rounded at 1024 * log2(e) before the maximum is subtracted would be off by 2^-14."""
+    cfg = dict(V=64, C=768, NL=1, NH=12, HD=64, FC=64, CTX=64, eps=0.0)
+    from test_oracle_gpt2 import split
+
+    rng = np.random.default_rng(T)
+    w = np.zeros(len(gpu.gpt2_random_weights(gpu.gpt2_cfg(**cfg), 1, 0.1)), np.float32)
+    wte, _, (L,), lnfw, _ = split(w, cfg)
+    for v in range(cfg["V"]):
+        wte[v] = rng.permutation(np.repeat([-1.0, 1.0], 384))
+    L["ln1w"][:] = L["ln2w"][:] = lnfw[:] = 1
+    L["qkvw"][np.arange(2304), np.concatenate([rng.permutation(768) for _ in range(3)])] = 1
+    L["qkvw"][0:1536:64] = 0                          # dim 0 of each head's q and k: 128 * 64 of the dot product
+    L["qkvb"][0:768:64], L["qkvb"][768:1536:64] = 128, 64
+    L["aow"][:] = np.eye(768)
+    ids = rng.integers(0, cfg["V"], T)
+    eng = gpu.Gpt2Engine(gpu.gpt2_cfg(**cfg), w)
+    got = eng.prefill([int(i) for i in ids])
+    eng.close()
+    x = wte[ids].astype(np.float64)
+    q, k, v = np.split(x @ L["qkvw"].T.astype(np.float64) + L["qkvb"], 3, 1)
+    sc = np.stack([(k[:, 64 * h:64 * h + 64] @ q[-1, 64 * h:64 * h + 64]) / 8 for h in range(12)])
+    p = np.exp(sc - sc.max(1, keepdims=True))
+    p /= p.sum(1, keepdims=True)
+    y = x[-1] + np.concatenate([p[h] @ v[:, 64 * h:64 * h + 64] for h in range(12)])
+    y -= y.mean()
+    want = y / np.sqrt((y * y).mean()) @ wte.T.astype(np.float64)
+    say("attention of large scores", T, np.abs(got - want).max() / np.abs(want).max())
+    assert np.abs(got - want).max() <= 2e-6 * np.abs(want).max()
+
+
 def test_engine_full_greedy_token_identical(gpu, og):
     cfg = gpu.gpt2_cfg()
     say("building GPT-2 124M random weights")
