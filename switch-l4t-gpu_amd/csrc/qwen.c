@@ -639,14 +639,25 @@ static int pf_chunk(sgpu_qwen *e, int c0, int Tc) {
  * the step record {ids[T-1], T-1} (so the on-device greedy loop continues from position T). */
 static int prefill_rows(sgpu_qwen *e, const int *ids, int T) {
     const sgpu_qwen_cfg *c = &e->cfg;
-    const int C = c->C, mm = T > MM_MIN_ROWS && mm_ok(c);
-    /* equal chunks (of whole 128-row tiles in the piece form) */
-    const int nchunk = mm ? (T + MM_ROWS - 1) / MM_ROWS : 1;
-    const int R = mm ? ((T + nchunk - 1) / nchunk + 127) / 128 * 128 : PF_ROWS;
+    const int C = c->C;
     void *s = (void *)e->stream;
-    int rc;
+    int rc, R = PF_ROWS, mm = T > MM_MIN_ROWS && mm_ok(c);
     if (!e->d_pf_ids) TRY(sgpu_malloc((void **)&e->d_pf_ids, (size_t)c->CTX * sizeof(int)));
-    TRY(mm ? mm_alloc(e, (R + 511) / 512 * 512) : pf_alloc(e));
+    if (mm) {
+        /* equal chunks of whole 128-row tiles; where the device has no room for their buffers, chunks
+         * of PF_ROWS rows, and then the form on fp32 tiles */
+        const int nchunk = (T + MM_ROWS - 1) / MM_ROWS;
+        R = ((T + nchunk - 1) / nchunk + 127) / 128 * 128;
+        if ((rc = mm_alloc(e, (R + 511) / 512 * 512)) && R > PF_ROWS) rc = mm_alloc(e, R = PF_ROWS);
+        if (rc == (int)hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            mm = 0;
+            R = PF_ROWS;
+        } else if (rc) {
+            return rc;
+        }
+    }
+    if (!mm) TRY(pf_alloc(e));
     hipError_t he = hipMemcpyAsync(e->d_pf_ids, ids, (size_t)T * sizeof(int), hipMemcpyHostToDevice, e->stream);
     if (he != hipSuccess) return (int)he;
     int Tc = 0;

@@ -263,6 +263,11 @@ def test_engine_prefill_attention_tiles(gpu, og, heads, T):
     fresh.close()
 
 
+def test_engine_prefill_second_piece_chunk(gpu, og):
+    """A prompt past the 4096 rows of one chunk: its second chunk's rows attend to the first's."""
+    test_engine_prefill_matches_golden(gpu, og, dict(cfg=dict(V=300, C=64, NL=2, NH=1, NKV=1, HD=64, FC=64, CTX=4200), T=4180))
+
+
 # The prompt products in fp16 pieces (from 65 rows on, 64-wide heads and whole 64-blocks): token
 # tiles of 64 and 128, column tiles of 64 to 256 and their remainders.
 @pytest.mark.parametrize("T", [65, 128, 129, 250])
@@ -271,6 +276,60 @@ def test_engine_prefill_pieces_tiles(gpu, og, sizes, T):
     NH, NKV, HD, FC = sizes
     test_engine_prefill_matches_golden(gpu, og, dict(
         cfg=dict(V=300, C=NH * HD, NL=2, NH=NH, NKV=NKV, HD=HD, FC=FC, CTX=260), T=T))
+
+
+# Prompt buffers: sgpu_malloc as the engine calls it, refusing what is larger than `limit` bytes but for
+# the split-K partials' 32 MB (or these as well), as a full device would.
+SHIM = """
+#include <stddef.h>
+extern int hipMalloc(void **p, size_t n);
+size_t limit = (size_t)-1;
+int partials_too = 0;
+int sgpu_malloc(void **p, size_t n) {
+    *p = 0;
+    if (n > limit && (partials_too || n != (32u << 20))) return 2;     /* hipErrorOutOfMemory */
+    return n ? hipMalloc(p, n) : 0;
+}
+"""
+SHIM_RUN = """
+import ctypes, sys
+sys.path.insert(0, sys.argv[2])
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)               # found before the library's own
+import numpy as np
+import sgpu
+cfg = dict(V=300, C=128, NL=2, NH=2, NKV=1, HD=64, FC=192, CTX=700)
+blob = sgpu.qwen_random_blob(sgpu.qwen_cfg(**cfg), seed=51, std=0.15)
+limit, too = ctypes.c_size_t.in_dll(shim, "limit"), ctypes.c_int.in_dll(shim, "partials_too")
+ids = [(7 * i) % 300 for i in range(600)]
+e = sgpu.QwenEngine(sgpu.qwen_cfg(**cfg), blob, sgpu.QWEN_PATH_FUSED)
+want = None
+for lim, t in ((-1, 0), (800000, 0), (800000, 1), (-1, 0)):
+    limit.value, too.value = 2**64 - 1, 0
+    e.close()
+    e = sgpu.QwenEngine(sgpu.qwen_cfg(**cfg), blob, sgpu.QWEN_PATH_FUSED)
+    e.prefill(ids[:70])
+    limit.value, too.value = lim % 2**64, t
+    got = e.prefill(ids).copy()
+    again = e.forward(5, 600).copy()
+    want = (got, again) if want is None else want
+    for g, w in zip((got, again), want):
+        assert np.abs(g - w).max() <= 1e-5 * np.abs(w).max(), (lim, t)
+    print("limit", lim, t, "equal" if np.array_equal(got, want[0]) else "close", flush=True)
+"""
+
+
+def test_engine_prefill_without_room_for_its_buffers(gpu, tmp_path):
+    """A prompt whose row buffers the device has no room for goes through in smaller chunks, then in the
+    form on fp32 tiles, with the logits of the whole one."""
+    (tmp_path / "shim.c").write_text(SHIM)
+    so = str(tmp_path / "shim.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", so, str(tmp_path / "shim.c"), "-L/opt/rocm/lib", "-lamdhip64",
+                    "-Wl,-rpath,/opt/rocm/lib"], check=True)
+    out = subprocess.run([sys.executable, "-c", SHIM_RUN, so, os.path.join(ROOT, "switch-l4t-gpu_amd")],
+                         capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0, out.stderr[-2000:]
+    forms = [line.split()[-1] for line in out.stdout.splitlines() if line.startswith("limit")]
+    assert len(forms) == 4 and forms[0] == forms[3] == "equal" and forms[2] == "close", out.stdout
 
 
 def test_engine_prefill_pieces_weight_codes(gpu, og):
