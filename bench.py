@@ -44,7 +44,7 @@ import sgpu  # noqa: E402
 
 METRIC = "SGEMM TFLOPS @4096³ + GEMV GB/s (% of HBM peak); decode tok/s"
 PEAK_FP32_MATRIX_TFLOPS = 157.3      # MI355X dense fp32 matrix
-PIECES_NOTE = ": fp32 operands cut exactly into three bf16 pieces, fp32 accumulation"
+PIECES_NOTE = ": fp32 operands cut into three bf16 pieces, the six largest piece products, fp32 accumulation"
 PEAK_PIECES_TFLOPS = 2500.0 / 6      # ... dense bf16 matrix over the six piece products of an fp32 product
 PEAK_HBM_GBPS = 8000.0               # MI355X HBM3E
 PROFILE_TRAFFIC = os.path.join(ROOT, "profiles", "traffic.json")

@@ -1102,6 +1102,7 @@ int sgpu_sgemm_opt(const float *A, const float *B, float *C, int M, int N, int K
     if (p == PLAN_SPLITK && sk_workspace(d, stream, &ws, &cnt) == SGPU_OK)    /* else: the unsplit member */
         return splitk_launch(d, A, B, C, M, N, K, S, ws, cnt, stream);
     if (plan_large(p) && pieces_taken(d, A, B, C, M, N, K, stream, &rc)) return rc;
+    /* 256 CUs take the piece form for all of sgemm_kwave128's plans of fewer than 2^20 tiles */
     if (p == PLAN_KWAVE128 && !(((uintptr_t)A | (uintptr_t)B) & 15))
         return sgemm_common(K_SGEMM_KWAVE128, "sgemm_kwave128", A, B, C, M, N, K, stream);
     if (p == PLAN_KWAVE && !(((uintptr_t)A | (uintptr_t)B) & 15)) return kwave_launch(0, A, B, C, M, N, K, stream);

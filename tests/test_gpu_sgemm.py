@@ -805,22 +805,27 @@ def test_kwave128_rejects_other_shapes(gpu):
     assert L.sgpu_sgemm_kwave128(dA.ptr, dB.ptr, dC.ptr, 0, 128, 64, None) == 0
 
 
-def test_opt_unaligned_kwave128_shape_takes_the_size_rule_member(gpu):
-    """sgpu_sgemm_opt plans sgemm_kwave128 for 2048^3; with A off 16-byte alignment it launches
-    the member the size rule picks (sgemm_tiled4), whose C it then equals bit for bit."""
+def test_opt_unaligned_kwave128_shape_takes_the_piece_form(gpu):
+    """sgpu_sgemm_opt plans sgemm_kwave128 for 2048^3 and runs its piece form, with A off 16-byte
+    alignment too: on random floats C equals sgpu_sgemm_pieces' bit for bit (and not the size-rule
+    member's, sgemm_tiled4)."""
     M = N = K = 2048
+    assert gpu.lib().sgpu_sgemm_opt_pieces(M, N, K, gpu.device_props().compute_units)
     rng = np.random.default_rng(2048)
-    A = rng.integers(-2, 3, (M, K)).astype(np.float32)
-    B = rng.integers(-2, 3, (K, N)).astype(np.float32)
+    A, B = rng.uniform(-1, 1, (M, K)).astype(np.float32), rng.uniform(-1, 1, (K, N)).astype(np.float32)
     C = run_sgemm(gpu, "sgpu_sgemm_opt", A, B, M, N, K, a_off=1)
-    D = run_sgemm(gpu, "sgpu_sgemm_tiled4", A, B, M, N, K, a_off=1)
-    assert np.array_equal(C, D)
+    assert np.array_equal(C, run_sgemm(gpu, "sgpu_sgemm_pieces", A, B, M, N, K, a_off=1))
+    assert not np.array_equal(C, run_sgemm(gpu, "sgpu_sgemm_tiled4", A, B, M, N, K, a_off=1))
 
 
 # sgpu_sgemm_pieces: tiles of 128x128 and 128x256 that end at M and N, k-slices of 32 with a last one
-# that overlaps, tails split over K (few tiles, or more tiles than CUs), odd float alignments.
+# that overlaps, odd float alignments; on 256 CUs one round or less, unsplit (128x128x32) and split
+# (255x513x993, 640x384x4097), several rounds unsplit (1100x8200x65, 2049x4111x200: too few slices), and
+# whole tiles with a split tail in one launch, 128x128 (2047x2049x2048: 256 tiles and 16, 16 ways) and
+# 128x256 (3073x3073x520: 256 tiles and 69, 3 ways; test_pieces_overlap_has_one_owner sees that
+# such tails are split).
 PIECES_CASES = [(128, 128, 32), (129, 128, 33), (128, 255, 63), (300, 257, 100), (255, 513, 31 * 32 + 1),
-                (640, 384, 4097), (2047, 2049, 130), (1100, 8200, 65), (2049, 4111, 200)]
+                (640, 384, 4097), (2047, 2049, 130), (1100, 8200, 65), (2049, 4111, 200), (2047, 2049, 2048), (3073, 3073, 520)]
 
 
 @pytest.mark.parametrize("a_off,b_off", [(0, 0), (1, 3)])
@@ -861,7 +866,8 @@ def test_pieces_overlap_has_one_owner(gpu, M, N, K):
     """Shapes whose last row or column of tiles is shifted back over its neighbour and where, on 256
     compute units, one of the two is split over K and the other is not: the elements of the unsplit
     tiles (of each tile's own rows and columns) equal bit for bit the product recorded on a stream
-    without a workspace, which splits no tile; the split ones differ from it somewhere."""
+    without a workspace, which splits no tile; the split ones differ from it somewhere.  Sampled rows of
+    both kinds are as close to float64 as fp32 sums are."""
     say(f"sgemm pieces overlap {M}x{N}x{K}")
     cus = gpu.device_props().compute_units
     kernel = gpu.lib().sgpu_sgemm_opt_pieces(M, N, K, cus)
@@ -886,6 +892,8 @@ def test_pieces_overlap_has_one_owner(gpu, M, N, K):
     for i, j in order[:full]:
         own[128 * i:128 * (i + 1), tn * j:tn * (j + 1)] = True
     assert 0 < full < ntm * ntn
+    rows = np.r_[0:M:M // 12, M - 130:M:13]
+    want = A[rows].astype(np.float64) @ B.astype(np.float64)
     for _ in range(3):
         dC.fill_bytes(0xFF)
         gpu.call("sgpu_sgemm_pieces", dA.ptr, dB.ptr, dC.ptr, M, N, K, None)
@@ -893,6 +901,7 @@ def test_pieces_overlap_has_one_owner(gpu, M, N, K):
         got = dC.to_host()
         assert np.array_equal(got[own], unsplit[own])
         assert not np.array_equal(got[~own], unsplit[~own])
+        assert np.linalg.norm(got[rows] - want) <= 1e-6 * np.linalg.norm(want)
 
 
 @pytest.mark.parametrize("scale_a,scale_b", [(1.0, 1.0), (1e-36, 1.0), (1.0, 1e-38), (1e-20, 1e-18), (1e30, 1e-30),

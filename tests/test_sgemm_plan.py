@@ -160,12 +160,14 @@ def test_piece_form_pinned_at_256_cus(M, N, K, kernel):
 
 
 def test_bench_traffic_record_covers_the_4096_member():
-    """bench.py reports the HBM traffic of the member sgpu_sgemm_opt launches at 4096^3 from
-    profiles/traffic.json under "<member>_4096"; a plan change that moves 4096^3 to another
-    member needs that member's PMC record, or the bench line's roofline.traffic goes null."""
+    """bench.py reports the HBM traffic of what sgpu_sgemm_opt launches at 4096^3 -- the piece kernel
+    sgpu_sgemm_opt_pieces names, else the planned member -- from profiles/traffic.json under
+    "<kernel>_4096"; a change that moves 4096^3 to another kernel needs that kernel's PMC record, or
+    the bench line's roofline.traffic goes null."""
     import json
 
-    name, _ = plan(4096, 4096, 4096, 256)
+    pieces = sgpu.lib().sgpu_sgemm_opt_pieces(4096, 4096, 4096, 256)
+    name = pieces.decode() if pieces else plan(4096, 4096, 4096, 256)[0]
     rec = json.load(open(os.path.join(ROOT, "profiles", "traffic.json")))
     assert f"{name}_4096" in rec
     assert rec[f"{name}_4096"] >= 3 * 4 * 4096 * 4096          # at least A, B and C once
