@@ -118,4 +118,40 @@ sgpu_probe_mfma(float* __restrict__ out, long long nout, int iters, float a0, fl
     }
 }
 
+// The rate of the 16-bit matrix cores: each wave issues iters x 32 v_mfma_f32_16x16x32 (fp16, or bf16
+// if bf != 0) on four independent accumulators, operands in registers -- pseudo-random in [-1, 1] if
+// rnd != 0, else zeros, whose power draw is lower -- and each thread stores one sum (out: a float per
+// launched thread).
+typedef _Float16 sgpu_f16x8_p __attribute__((ext_vector_type(8)));
+typedef __bf16 sgpu_bf16x8_p __attribute__((ext_vector_type(8)));
+__global__ void __launch_bounds__(256) sgpu_probe_mfma16(float* __restrict__ out, int iters, int bf, int rnd) {
+    sgpu_f16x8_p a, b;
+    sgpu_bf16x8_p a2, b2;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const unsigned h = (threadIdx.x * 8u + i + blockIdx.x * 77u) * 2654435761u;
+        const float v = rnd ? (float)((int)(h >> 8) % 2001 - 1000) / 1000.0f : 0.0f;
+        a[i] = (_Float16)v;
+        b[i] = (_Float16)(v * 0.7f);
+        a2[i] = (__bf16)v;
+        b2[i] = (__bf16)(v * 0.7f);
+    }
+    sgpu_f32x4 acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) acc[i] = sgpu_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (bf) {
+        for (int it = 0; it < iters; it++)
+#pragma unroll
+            for (int u = 0; u < 32; u++) acc[u % 4] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, b2, acc[u % 4], 0, 0, 0);
+    } else {
+        for (int it = 0; it < iters; it++)
+#pragma unroll
+            for (int u = 0; u < 32; u++) acc[u % 4] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, acc[u % 4], 0, 0, 0);
+    }
+    float s = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) s += (acc[i][0] + acc[i][1]) + (acc[i][2] + acc[i][3]);
+    out[(size_t)blockIdx.x * 256 + threadIdx.x] = s;
+}
+
 }  // extern "C"

@@ -10,6 +10,8 @@
  *            one wave per SIMD, iters x 16 fp32 32x32x2 MFMAs per wave with operands in
  *            registers, then a 4 MB store: iters 0 (launch and store only) to 512.  At iters 32
  *            each SIMD issues the MFMA count of a 1024^3 SGEMM spread over the 256 CUs.
+ *   mfma16 -- sgpu_probe_mfma16 on 512 blocks, two waves per SIMD, 1000 x 32 fp16 or bf16 16x16x32 MFMAs
+ *            per wave, on pseudo-random operands and on zeros: the rate the piece forms can reach
  *   sgemm -- sgpu_sgemm_opt at 1024^3 (sgemm_kwave), 768x1024x1024 and 1023x1025x997
  *            (sgemm_kwave_edge) on integer inputs, each result checked exactly before timing.
  */
@@ -58,19 +60,23 @@ static double time_graph(hipGraphExec_t ge, double warm_s, int reps) {
     return best * 1e3 / LAUNCHES;
 }
 
-static double mfma_leg(hipFunction_t f, float *out, long long nout, int iters, double warm_s, int reps) {
-    float a0 = 1.0f, b0 = 1.0f;
-    void *kp[] = {&out, &nout, &iters, &a0, &b0};
+static double probe_leg(hipFunction_t f, int blocks, void **kp, double warm_s, int reps) {
     hipGraph_t g;
     hipGraphExec_t ge;
     CHK(hipStreamBeginCapture(stream, hipStreamCaptureModeRelaxed));
-    for (int l = 0; l < LAUNCHES; l++) CHK(hipModuleLaunchKernel(f, BLOCKS, 1, 1, 256, 1, 1, 0, stream, kp, NULL));
+    for (int l = 0; l < LAUNCHES; l++) CHK(hipModuleLaunchKernel(f, blocks, 1, 1, 256, 1, 1, 0, stream, kp, NULL));
     CHK(hipStreamEndCapture(stream, &g));
     CHK(hipGraphInstantiate(&ge, g, NULL, NULL, 0));
     const double us = time_graph(ge, warm_s, reps);
     CHK(hipGraphExecDestroy(ge));
     CHK(hipGraphDestroy(g));
     return us;
+}
+
+static double mfma_leg(hipFunction_t f, float *out, long long nout, int iters, double warm_s, int reps) {
+    float a0 = 1.0f, b0 = 1.0f;
+    void *kp[] = {&out, &nout, &iters, &a0, &b0};
+    return probe_leg(f, BLOCKS, kp, warm_s, reps);
 }
 
 /* sgpu_sgemm_opt on integer inputs in [-2, 2]: the result is checked exactly (every partial
@@ -126,8 +132,9 @@ int main(int argc, char **argv) {
     const void *co = sgpu_code_object("sgpu_probe", &colen);
     if (!co) { fprintf(stderr, "no sgpu_probe code object\n"); return 1; }
     hipModule_t mod;
-    hipFunction_t f;
+    hipFunction_t f, f16;
     CHK(hipModuleLoadData(&mod, co));
+    CHK(hipModuleGetFunction(&f16, mod, "sgpu_probe_mfma16"));
     CHK(hipModuleGetFunction(&f, mod, "sgpu_probe_mfma"));
     CHK(hipStreamCreate(&stream));
     CHK(hipEventCreate(&ev0));
@@ -149,6 +156,16 @@ int main(int argc, char **argv) {
         fprintf(stderr, "mfma probe, %4d MFMAs per wave: %8.3f us per launch (issue time at 2.4 GHz %.3f us)\n",
                 (int)per_simd, us, ideal);
         printf("%s{\"mfma_per_wave\":%d,\"us\":%.3f,\"issue_us_2p4ghz\":%.3f}", i ? "," : "", (int)per_simd, us, ideal);
+    }
+    printf("],\"mfma16\":[");
+    for (int i = 0; i < 4; i++) {
+        int bf = i & 1, rnd = i >> 1, n = 1000, blocks = 2 * BLOCKS;
+        void *kp[] = {&out, &n, &bf, &rnd};
+        const double us = probe_leg(f16, blocks, kp, warm_s, reps);
+        const double tf = 4.0 * blocks * 32 * n * 2 * 16 * 16 * 32 / us / 1e6;
+        fprintf(stderr, "%s 16x16x32 MFMAs on %s: %.0f TFLOP/s\n", bf ? "bf16" : "fp16", rnd ? "random operands" : "zeros", tf);
+        printf("%s{\"type\":\"%s\",\"operands\":\"%s\",\"tflops\":%.0f}", i ? "," : "", bf ? "bf16" : "fp16",
+               rnd ? "random" : "zeros", tf);
     }
     printf("]");
 
