@@ -103,9 +103,10 @@ int sgpu_event_elapsed_ms(float *ms, void *start, void *stop);
 
 /* ---- code objects (the PTX modules' role: switch_gpu.ptx, gemv.ptx, gpt2.ptx, qwen.ptx) ----
  * Returns the embedded gfx950 ELF code object named "switch_gpu", "gemv", "gpt2_kernels",
- * "qwen_kernels", "sgpu_tuned", "sgpu_decode" or "sgpu_probe" (and its size), ready for
- * hipModuleLoadData; NULL if the name is unknown.  The first four export the reference's
- * kernel names and arguments; "sgpu_probe" holds the measurement kernels of bin/decode_floor. */
+ * "qwen_kernels", "sgpu_tuned", "sgpu_decode", "sgpu_prefill", "sgpu_pieces" or "sgpu_probe" (and
+ * its size), ready for hipModuleLoadData; NULL if the name is unknown.  The first four export the
+ * reference's kernel names and arguments; "sgpu_probe" holds the measurement kernels of
+ * bin/decode_floor and bin/sgemm_floor. */
 const void *sgpu_code_object(const char *name, size_t *size);
 
 /* Launch geometry the launchers use for a reference-named kernel at a given shape

@@ -1,21 +1,21 @@
 // sgpu_prefill.hip -- the Qwen2.5 prompt's products on the fp16 matrix cores (gfx950).
 //
 // The layer weights are fp16, so only x has to be cut to fit the fp16 matrix instructions, and
-// it is cut without loss: the kernels that produce an x (RMSNorm, attention, SwiGLU) write it as
+// it keeps its 24 bits: the kernels that produce an x (RMSNorm, attention, SwiGLU) write it as
 // three fp16 pieces x * 2^s = p0 + p1 + p2 (11 + 11 + 2 of the 24 mantissa bits), s one power of
 // two per row and 64 consecutive values, chosen so that the largest of them lies in
 // [2^14, 2^15).  Every product of a weight and a piece is exact in the fp32 accumulators, and
 // an fp32 dot product costs three fp16 MFMAs instead of sixteen fp32 ones' time.  A value less
 // than 2^-16 of its block's largest keeps fewer than 24 bits: the pieces' error is at most
-// 2^-40 of the block's largest value.
+// 2^-39 of the block's largest value (half an fp16 subnormal step, 2^-25, over 2^14).
 //
 // Piece layout ("planes"): row t holds K codes of p0, K of p1, K of p2; beside them one float
 // 2^-s per row and 64-block.  Non-finite values go to p0 as they are (p1 = p2 = 0) and s is
 // chosen over the finite ones.
 //
 // Measured against the same layers on fp32 MFMA tiles (sgpu_pf_gemm, 32x32 per block): a prompt
-// of 500 rows of the Qwen2.5-0.5B sizes 6.08 -> 3.30 ms, of 3001 rows 39.5 -> 11.5 ms; distance
-// of the logits from a 64-bit forward 1.1e-6 -> 6.4e-7 and 9.3e-7 -> 8.0e-7.
+// of 500 rows of the Qwen2.5-0.5B sizes 6.08 -> 3.30 ms, of 3001 rows 39.5 -> 11.1-11.5 ms; distance
+// of the logits from a 64-bit forward 1.1e-6 -> 6.2e-7 and 9.3e-7 -> 7.0e-7.
 //
 // This code object keeps fp16 subnormals (the pieces use them).  The reference reads subnormal
 // weights as +0: the engine clears those codes once, where it uploads the weights
@@ -75,8 +75,8 @@ enum { EPI_STORE, EPI_SWIGLU };
 // Y[t][n] = X[t] . W[n] + bias?[n] (EPI_STORE; accum != 0: added to Y), or silu(gate) * up as
 // pieces for the next product (EPI_SWIGLU: W holds N gate rows, then N up rows).
 //
-// Bound: the matrix cores, and below some 1000 rows the steps' loads.  (These cores reach 1.7-2.0
-// PFLOP/s on dense operands, 2.5 on zeros; gate|up at 3001 rows runs at 1.04 PFLOP/s of piece
+// Bound: the matrix cores, and below some 1000 rows the steps' loads.  (These cores reach 2.0
+// PFLOP/s on random operands, 2.26 on zeros, by bin/sgemm_floor; gate|up at 3001 rows runs at 1.04 PFLOP/s of piece
 // products, 1.4 with its loads taken out.)  A block of 2x2 waves computes 64*TF tokens x 64*NF weight rows, a
 // wave 32*TF x 32*NF of them in 16x16 tiles.  Per step of 64 k the block's pieces and weights go straight into
 // LDS (16 bytes a lane, no registers; a row's eight 16-byte chunks are stored at chunk ^ (row / 2
